@@ -157,6 +157,35 @@ typedef struct lime_ragged_batch {
  */
 int lime_lindblad_rk4_ragged(const lime_ragged_batch* r, const lime_step_params* p, void* stream);
 
+/*
+ * Workgroup lists for lime_lindblad_rk4_ragged_tiles: DEVICE arrays of (instance, item)
+ * int32 pairs, one per workgroup.  With tpd = ceil(n / tile), tiles = tpd^2:
+ *   stage: every instance's tiles 0 .. tiles - 1 (row-major), each once;
+ *   left:  every instance's k * tiles + t for k < n_dense, t < tiles, each once.
+ * Entry b runs on XCD b % 8: keep an instance's entries at one residue, so its operands stay
+ * in one L2.  An entry whose instance is negative is skipped (padding).
+ */
+typedef struct lime_ragged_tiles {
+  int32_t tile;                  /* tile edge: 32 or 64                                  */
+  int32_t stage_count;
+  int32_t left_count;            /* 0 when no instance has dense jump operators          */
+  int32_t reserved;
+  const int32_t* stage;
+  const int32_t* left;
+} lime_ragged_tiles;
+
+/*
+ * lime_lindblad_rk4_ragged with one launch per phase of an RK4 stage (the products T_k = L_k S
+ * of all instances, then the stage of all instances) instead of one persistent launch: every
+ * tile is a workgroup, so few or large instances still fill the GPU.  The same results, bit
+ * for bit.  r->variant, max_groups, order and queue are not used (order and queue may be
+ * NULL).  The caller guarantees that the lists and the offsets address its pools.
+ * Capturable in a HIP graph (no host synchronisation, no allocation).
+ * Replaces the same loop of lime as lime_lindblad_rk4_ragged.
+ */
+int lime_lindblad_rk4_ragged_tiles(const lime_ragged_batch* r, const lime_ragged_tiles* t, const lime_step_params* p,
+                                   void* stream);
+
 /* Number of launch shapes of lime_lindblad_rk4_ragged (the autotuner times each one). */
 int lime_ragged_variants(void);
 

@@ -28,6 +28,7 @@ EXPORTS = (
     "lime_lindblad_rk4",
     "lime_lindblad_rk4_noalloc",
     "lime_lindblad_rk4_ragged",
+    "lime_lindblad_rk4_ragged_tiles",
     "lime_ragged_variants",
     "lime_lindblad_max_n",
     "lime_lindblad_workspace_bytes",
@@ -104,6 +105,17 @@ class RaggedBatch(ctypes.Structure):
     ]
 
 
+class RaggedTiles(ctypes.Structure):
+    _fields_ = [
+        ("tile", ctypes.c_int32),
+        ("stage_count", ctypes.c_int32),
+        ("left_count", ctypes.c_int32),
+        ("reserved", ctypes.c_int32),
+        ("stage", ctypes.c_void_p),
+        ("left", ctypes.c_void_p),
+    ]
+
+
 class StepParams(ctypes.Structure):
     _fields_ = [
         ("dt", ctypes.c_double),
@@ -138,6 +150,10 @@ def load(path=LIB_PATH):
         lib.lime_lindblad_rk4_ragged.argtypes = [ctypes.POINTER(RaggedBatch),
                                                  ctypes.POINTER(StepParams), ctypes.c_void_p]
         lib.lime_lindblad_rk4_ragged.restype = ctypes.c_int
+        lib.lime_lindblad_rk4_ragged_tiles.argtypes = [ctypes.POINTER(RaggedBatch),
+                                                       ctypes.POINTER(RaggedTiles),
+                                                       ctypes.POINTER(StepParams), ctypes.c_void_p]
+        lib.lime_lindblad_rk4_ragged_tiles.restype = ctypes.c_int
         lib.lime_ragged_variants.argtypes = []
         lib.lime_ragged_variants.restype = ctypes.c_int
         lib.lime_lindblad_max_n.argtypes = [ctypes.c_int32, ctypes.c_int32]

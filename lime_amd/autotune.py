@@ -16,6 +16,8 @@ import threading
 
 import torch
 
+from . import _lib
+
 _lock = threading.Lock()
 _CACHE_PATH = os.environ.get("LIME_TUNE_CACHE") or os.path.join(
     os.environ.get("XDG_CACHE_HOME") or os.path.join(os.path.expanduser("~"), ".cache"),
@@ -45,6 +47,12 @@ def _save():
         pass
 
 
+def _version():
+    """The library's version: a build's choices are not taken over by another build, whose
+    variants may be other kernels."""
+    return _lib.load().lime_version().decode()
+
+
 def _bucket(batch):
     b = 1
     while b < batch:
@@ -53,7 +61,7 @@ def _bucket(batch):
 
 
 def key_of(prop, n_eops=0):
-    return (f"n{prop.n}:kd{prop.n_dense}:{prop.precision}:b{_bucket(prop.batch)}"
+    return (f"{_version()}:n{prop.n}:kd{prop.n_dense}:{prop.precision}:b{_bucket(prop.batch)}"
             f":e{int(n_eops > 0)}:t{int(prop.force_tiled)}")
 
 
@@ -111,7 +119,7 @@ def tune(prop, rho, dt, steps=4, n_eops=0, force=False, verbose=False, eops_t=No
 def tune_ragged(rb, dt, steps=2, force=False, verbose=False):
     """Pick the fastest persistent launch shape of a ``RaggedLindblad`` batch (states are
     restored afterwards); cached per (instance count, sum of n^3 (1 + K_d))."""
-    key = f"ragged:c{rb.count}:w{int(rb.work_units)}"
+    key = f"{_version()}:ragged:c{rb.count}:w{int(rb.work_units)}"
     with _lock:
         cache = _load()
         if not force and key in cache:
@@ -120,7 +128,7 @@ def tune_ragged(rb, dt, steps=2, force=False, verbose=False):
     saved = rb.rho.clone()
     times = {}
     stream = torch.cuda.current_stream(rb.dev)
-    for v in range(rb.variants()):
+    for v in range(rb.launches()):
         rb.variant = v
         rb.step(dt, 1)                                   # warm-up
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)

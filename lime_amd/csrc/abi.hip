@@ -201,7 +201,7 @@ extern "C" {
 
 const char* lime_last_error(void) { return g_last_error.c_str(); }
 
-const char* lime_version(void) { return "lime_hip 0.2 (gfx950)"; }
+const char* lime_version(void) { return "lime_hip 0.3 (gfx950)"; }
 
 int lime_lindblad_max_n(int32_t n_dense, int32_t flags) {
   if ((flags & LIME_F_PREC_MASK) != LIME_F_PREC_FP32) return 0;
@@ -296,6 +296,35 @@ int lime_lindblad_rk4_ragged(const lime_ragged_batch* r, const lime_step_params*
   a.queue = static_cast<unsigned*>(r->queue);
   hipError_t e = lime::ragged_run(a, r->variant, r->max_groups, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "lime_lindblad_rk4_ragged launch");
+  return LIME_OK;
+}
+
+int lime_lindblad_rk4_ragged_tiles(const lime_ragged_batch* r, const lime_ragged_tiles* t, const lime_step_params* p,
+                                   void* stream) {
+  const std::string name = "lime_lindblad_rk4_ragged_tiles";
+  if (r == nullptr || t == nullptr || p == nullptr) return fail(LIME_ERR_ARG, name + ": null descriptor");
+  if (r->count < 0 || p->nsteps < 0) return fail(LIME_ERR_ARG, name + ": count and nsteps must be >= 0");
+  if (r->count == 0 || p->nsteps == 0) return LIME_OK;
+  if (t->tile != 32 && t->tile != 64) return fail(LIME_ERR_ARG, name + ": tile must be 32 or 64");
+  if (t->stage_count < 1 || t->left_count < 0 || !t->stage || (t->left_count > 0 && !t->left))
+    return fail(LIME_ERR_ARG, name + ": stage and left lists are required");
+  if (!r->inst || !r->ops || !r->rho || !r->work) return fail(LIME_ERR_ARG, name + ": inst, ops, rho and work are required");
+  lime::RaggedArgs a = {};
+  a.inst = reinterpret_cast<const lime::RaggedInstance*>(r->inst);
+  a.count = r->count;
+  a.nsteps = p->nsteps;
+  a.dt = p->dt;
+  a.ops = static_cast<const float2*>(r->ops);
+  a.rho = static_cast<double2*>(r->rho);
+  a.work = static_cast<float2*>(r->work);
+  lime::RaggedTiles l;
+  l.tile = t->tile;
+  l.stage_count = t->stage_count;
+  l.left_count = t->left_count;
+  l.stage = reinterpret_cast<const int2*>(t->stage);
+  l.left = reinterpret_cast<const int2*>(t->left);
+  hipError_t e = lime::ragged_tiles_run(a, l, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "lime_lindblad_rk4_ragged_tiles launch");
   return LIME_OK;
 }
 

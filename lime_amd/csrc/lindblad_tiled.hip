@@ -1106,6 +1106,28 @@ __device__ __forceinline__ RaggedInstance uniform_instance(const RaggedInstance&
   return u;
 }
 
+// The per-stage kernels' arguments of one instance (its operators, state and workspace);
+// the stage and its operands s_cur / s_next are set by the caller.
+__device__ __forceinline__ TiledArgs instance_args(const RaggedArgs& r, const RaggedInstance& in) {
+  TiledArgs a = {};
+  a.batch = 1;
+  a.n = in.n;
+  a.nc = in.n;
+  a.group = 1;
+  a.n_dense = in.n_dense;
+  a.dt = r.dt;
+  a.rec = -1;
+  a.heff = r.ops + in.heff;
+  a.dmat = in.dmat >= 0 ? r.ops + in.dmat : nullptr;
+  a.lops = in.n_dense > 0 ? r.ops + in.lops : nullptr;
+  a.rho = r.rho + in.rho;
+  float2* s0 = r.work + in.work;
+  const size_t nn = (size_t)in.n * in.n;
+  a.inc = s0 + 2 * nn;
+  a.tbuf = s0 + 3 * nn;
+  return a;
+}
+
 template <int TILE, int SG, int MINW>
 __global__ void __launch_bounds__(256 * SG) __attribute__((amdgpu_waves_per_eu(MINW)))
 lindblad_ragged_persistent(RaggedArgs r) {
@@ -1124,22 +1146,9 @@ lindblad_ragged_persistent(RaggedArgs r) {
     const RaggedInstance in = uniform_instance(r.inst[__builtin_amdgcn_readfirstlane(r.order[item])]);
     const int n = in.n;
     const size_t nn = (size_t)n * n;
-    TiledArgs a = {};
-    a.batch = 1;
-    a.n = n;
-    a.nc = n;
-    a.group = 1;
-    a.n_dense = in.n_dense;
-    a.dt = r.dt;
-    a.rec = -1;
-    a.heff = r.ops + in.heff;
-    a.dmat = in.dmat >= 0 ? r.ops + in.dmat : nullptr;
-    a.lops = in.n_dense > 0 ? r.ops + in.lops : nullptr;
-    a.rho = r.rho + in.rho;
+    TiledArgs a = instance_args(r, in);
     C* s0 = r.work + in.work;
     C* s1 = s0 + nn;
-    a.inc = s1 + nn;
-    a.tbuf = s1 + 2 * nn;
     for (size_t i = threadIdx.x; i < nn; i += blockDim.x) s0[i] = make_float2((float)a.rho[i].x, (float)a.rho[i].y);
     __syncthreads();
     const int tiles = tiles_per_dim(n, TILE) * tiles_per_dim(n, TILE);
@@ -1189,6 +1198,96 @@ lindblad_ragged_persistent(RaggedArgs r) {
     atomicExch(r.queue, 0u);
     atomicExch(r.queue + 1, 0u);
   }
+}
+
+// ---- uneven batches, one launch per phase of a stage
+// The persistent launch above keeps an instance on one compute unit, so its time is that of
+// the largest instance whenever the instances do not outnumber the compute units several
+// times over.  Here every tile of every instance is a workgroup of its own: a stage is one
+// launch over the tiles of all products T_k = L_k S and one over the tiles of the stage, the
+// kernel boundary is the barrier.  The workgroup -> (instance, tile) lists come from the
+// caller, interleaved over the XCDs (list entry b runs on XCD b % 8): an instance's tiles stay
+// on one XCD, whose L2 then holds its operands, and each XCD gets the same share of the work.
+// The tile code is the persistent kernel's, term by term, so the results are the same bits.
+// Measured, us per step (persistent at its best launch shape / per phase): 256 instances of
+// n = 16..256 with 4 dense L 12100 / 3450 (114 TFLOP/s canonical), 1024 of them 16300 /
+// 12100, 16 of them 7100 / 320.  The persistent launch stays ahead where every instance is
+// one tile and the phases are launch-bound: 2048 of n = 16 35 / 44, 2048 of n = 32 with two
+// L 177 / 217, one of n = 24 38 / 46.  The autotuner picks per batch.
+__device__ __forceinline__ bool ragged_entry(const RaggedArgs& r, const int2* list, RaggedInstance& in, int& item) {
+  const int2 e = list[blockIdx.x];
+  const int i = __builtin_amdgcn_readfirstlane(e.x);
+  item = __builtin_amdgcn_readfirstlane(e.y);
+  if (i < 0) return false;                    // padding of the shorter XCD lists
+  in = uniform_instance(r.inst[i]);
+  return true;
+}
+
+// s0 = rho in the operand precision, one workgroup per stage tile
+template <int TILE>
+__global__ void __launch_bounds__(256) ragged_init(RaggedArgs r, const int2* list) {
+  RaggedInstance in;
+  int t;
+  if (!ragged_entry(r, list, in, t)) return;
+  const int n = in.n, tpd = tiles_per_dim(n, TILE);
+  const int row0 = (t / tpd) * TILE, col0 = (t % tpd) * TILE;
+  const double2* rho = r.rho + in.rho;
+  float2* s0 = r.work + in.work;
+  for (int e = threadIdx.x; e < TILE * TILE; e += 256) {
+    const int i = row0 + e / TILE, j = col0 + e % TILE;
+    if (i < n && j < n) {
+      const double2 x = rho[(size_t)i * n + j];
+      s0[(size_t)i * n + j] = make_float2((float)x.x, (float)x.y);
+    }
+  }
+}
+
+// T_k = L_k S of stage `st`: list items k * tiles + tile
+template <int TILE>
+__global__ void __launch_bounds__(256) lindblad_ragged_left(RaggedArgs r, const int2* list, int st) {
+  __shared__ __align__(16) unsigned char smem[smem_bytes<TILE, float, 0>()];
+  RaggedInstance in;
+  int item;
+  if (!ragged_entry(r, list, in, item)) return;
+  const int tpd = tiles_per_dim(in.n, TILE), tiles = tpd * tpd;
+  TiledArgs a = instance_args(r, in);
+  a.s_cur = r.work + in.work + (st % 2 == 0 ? 0 : (size_t)in.n * in.n);
+  const Geo g = geometry<TILE>(in.n, item % tiles, threadIdx.x);
+  left_tile<TILE, float, 0, true>(a, 0, item / tiles, g, smem);
+}
+
+// One RK4 stage: list items are the tiles
+template <int TILE>
+__global__ void __launch_bounds__(256) lindblad_ragged_stage(RaggedArgs r, const int2* list, int st) {
+  __shared__ __align__(16) unsigned char smem[smem_bytes<TILE, float, 0>()];
+  RaggedInstance in;
+  int tile;
+  if (!ragged_entry(r, list, in, tile)) return;
+  const int n = in.n;
+  TiledArgs a = instance_args(r, in);
+  float2* s0 = r.work + in.work;
+  float2* s1 = s0 + (size_t)n * n;
+  a.stage = st;
+  a.s_cur = (st % 2 == 0) ? s0 : s1;
+  a.s_next = (st % 2 == 0) ? s1 : s0;
+  const Geo g = geometry<TILE>(n, tile, threadIdx.x);
+  constexpr int BW = TILE / 32;
+  floatx4 cr[BW][BW], ci[BW][BW];
+#pragma unroll
+  for (int p = 0; p < BW; ++p)
+#pragma unroll
+    for (int q = 0; q < BW; ++q) cr[p][q] = ci[p][q] = floatx4{0.f, 0.f, 0.f, 0.f};
+  generator_gemms<TILE, float, 0, true>(a, 0, g, smem, cr, ci, 0, n);
+#pragma unroll
+  for (int p = 0; p < BW; ++p)
+#pragma unroll
+    for (int q = 0; q < BW; ++q)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int i = g.row0 + g.wr * (TILE / 2) + p * 16 + CT<float>::row(g.lg, v);
+        const int j = g.col0 + g.wc * (TILE / 2) + q * 16 + g.lr;
+        if (i < n && j < n) stage_elem<float>(a, 0, 0, (size_t)i * n + j, cr[p][q][v], ci[p][q][v]);
+      }
 }
 
 // Gradient contractions of an adjoint stage operator kappa with a forward stage operator
@@ -1691,6 +1790,23 @@ hipError_t ragged_run(const RaggedArgs& r, int variant, int max_groups, hipStrea
     case 4: return ragged_launch_shape<32, 1, 4>(r, max_groups, stream);   // 4 waves, 4 per CU
     default: return hipErrorInvalidValue;
   }
+}
+
+template <int TILE>
+static hipError_t ragged_tiles_impl(const RaggedArgs& r, const RaggedTiles& t, hipStream_t stream) {
+  if (t.stage_count == 0) return hipSuccess;
+  hipLaunchKernelGGL(ragged_init<TILE>, dim3(t.stage_count), dim3(256), 0, stream, r, t.stage);
+  for (int s = 0; s < r.nsteps; ++s)
+    for (int st = 0; st < 4; ++st) {
+      if (t.left_count > 0)
+        hipLaunchKernelGGL(lindblad_ragged_left<TILE>, dim3(t.left_count), dim3(256), 0, stream, r, t.left, st);
+      hipLaunchKernelGGL(lindblad_ragged_stage<TILE>, dim3(t.stage_count), dim3(256), 0, stream, r, t.stage, st);
+    }
+  return hipGetLastError();
+}
+
+hipError_t ragged_tiles_run(const RaggedArgs& r, const RaggedTiles& t, hipStream_t stream) {
+  return t.tile == 64 ? ragged_tiles_impl<64>(r, t, stream) : ragged_tiles_impl<32>(r, t, stream);
 }
 
 hipError_t tiled_run(TiledArgs a, int nsteps, int step_offset, int nout, void* work, hipStream_t stream,

@@ -111,6 +111,15 @@ struct RaggedArgs {
   float2* work;
   unsigned* queue;              // [2]: next item, finished workgroups (zero between launches)
 };
+// Workgroup lists of the per-phase launches: (instance, tile) of a stage, (instance,
+// k * tiles + tile) of the products T_k = L_k S; an entry with instance < 0 is padding.
+struct RaggedTiles {
+  int tile;                     // tile edge, 32 or 64
+  int stage_count, left_count;
+  const int2* stage;
+  const int2* left;
+};
+hipError_t ragged_tiles_run(const RaggedArgs& r, const RaggedTiles& t, hipStream_t stream);
 int ragged_variants();
 hipError_t ragged_run(const RaggedArgs& r, int variant, int max_groups, hipStream_t stream);
 hipError_t contract_launch(const ContractArgs& c, hipStream_t stream);

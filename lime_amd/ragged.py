@@ -1,14 +1,19 @@
 """Ragged batches: many independent Lindblad systems of uneven dimension.
 
 lime propagates one system at a time (oqs.py:1590-1688).  ``RaggedLindblad`` takes a list
-of instances of different n and advances all of them together, in ONE kernel launch
-(``lime_lindblad_rk4_ragged``): the instances are packed into three pools (complex64
-operators, complex128 states, complex64 per-stage workspace), ordered by cost
-n^3 (1 + K_d) (largest first), and a persistent grid of workgroups drains that order
-through an atomic queue, each instance on one workgroup for every step of the call.  The
-launch shape (tile edge, tile groups per workgroup) comes from the autotuner
-(``lime_amd.autotune.tune_ragged``); ``capture``/``run`` put the launch in a hipGraph
-(torch.cuda.CUDAGraph) and replay it.
+of instances of different n and advances all of them together.  The instances are packed
+into three pools (complex64 operators, complex128 states, complex64 per-stage workspace).
+Two organisations step them, with the same results bit for bit:
+
+* one persistent launch (``lime_lindblad_rk4_ragged``): a grid of workgroups drains the
+  instances, ordered by cost n^3 (1 + K_d), through an atomic queue, each instance on one
+  workgroup for every step of the call;
+* one launch per phase of a stage (``lime_lindblad_rk4_ragged_tiles``): every tile of every
+  instance is a workgroup of its own, so few or large instances fill the GPU too.
+
+The autotuner (``lime_amd.autotune.tune_ragged``) times both, with their launch shapes, on
+the batch; ``capture``/``run`` put the launches in a hipGraph (torch.cuda.CUDAGraph) and
+replay it.
 
 ``RaggedClasses`` is the earlier organisation, kept as the comparison point: size classes,
 one operator batch each on the per-class fused kernels, all captured into one graph.
@@ -24,6 +29,10 @@ import torch
 
 from . import autotune
 from .propagator import LindbladPropagator, device
+
+
+XCDS = 8                 # accelerator dies of the GPU, each with its own L2
+TILE_EDGES = (32, 64)    # output tiles of the per-phase launches
 
 
 def fold_host(inst):
@@ -51,8 +60,42 @@ def fold_host(inst):
     return H - 0.5j * G, D, dense
 
 
+def tile_lists(sizes, kd, cost, edge):
+    """(stage, left) workgroup lists of ``lime_lindblad_rk4_ragged_tiles``: int32 (count, 2)
+    arrays of (instance, tile) and (instance, k * tiles + tile).
+
+    Instances are dealt to the 8 XCDs, the most expensive first, each to the XCD with the
+    least work so far; list entry b belongs to XCD b % 8, so an instance's tiles share one
+    L2 and every XCD starts with its largest instances.  (-1, -1) pads the shorter lists."""
+    tiles = ((np.asarray(sizes, dtype=np.int64) + edge - 1) // edge) ** 2
+    load = np.zeros(XCDS)
+    mine = [[] for _ in range(XCDS)]
+    for i in np.argsort(-np.asarray(cost), kind="stable"):
+        x = int(np.argmin(load))
+        load[x] += cost[i]
+        mine[x].append(i)
+
+    def interleave(items):
+        per = []
+        for ids in mine:
+            ids = np.asarray(ids, dtype=np.int64)
+            c = items[ids]
+            e = np.empty((int(c.sum()), 2), dtype=np.int32)
+            e[:, 0] = np.repeat(ids, c)
+            e[:, 1] = np.arange(len(e)) - np.repeat(np.cumsum(c) - c, c)
+            per.append(e)
+        out = np.full((max(len(e) for e in per), XCDS, 2), -1, dtype=np.int32)
+        for x, e in enumerate(per):
+            out[:len(e), x] = e
+        return out.reshape(-1, 2)
+
+    return interleave(tiles), interleave(tiles * np.asarray(kd, dtype=np.int64))
+
+
 class RaggedLindblad:
-    """One persistent launch for a list of instances of uneven n (FP32 MFMA, FP64 state)."""
+    """A list of instances of uneven n advanced together (FP32 MFMA, FP64 state): one
+    persistent launch, or one launch per phase of a stage, whichever the autotuner measured
+    faster on the batch (the same results, bit for bit)."""
 
     def __init__(self, instances, tune=True, dt_tune=0.01, verbose=False, max_groups=0):
         from . import _lib
@@ -101,6 +144,8 @@ class RaggedLindblad:
         self.order = torch.as_tensor(order, device=self.dev)
         self.queue = torch.zeros(2, dtype=torch.int32, device=self.dev)
         self.max_groups = int(max_groups)
+        self.cost = cost
+        self._lists = {}
         self.variant = 0
         self.graph = None
         if tune:
@@ -108,7 +153,25 @@ class RaggedLindblad:
             autotune.tune_ragged(self, dt_tune, verbose=verbose)
 
     def variants(self):
+        """Launch shapes of the persistent kernel."""
         return int(self._lib.lime_ragged_variants())
+
+    def launches(self):
+        """Values of ``variant`` the autotuner times: the persistent launch shapes, then one
+        launch per phase of a stage with 32 x 32 and with 64 x 64 tiles (not with a cap on
+        the persistent workgroups)."""
+        return self.variants() + (0 if self.max_groups else len(TILE_EDGES))
+
+    def _tile_lists(self, edge):
+        """Device lists of ``lime_lindblad_rk4_ragged_tiles`` for a tile edge (made once)."""
+        if edge not in self._lists:
+            from . import _lib
+            stage, left = (torch.as_tensor(x, device=self.dev) for x in tile_lists(self.sizes, self.kd, self.cost, edge))
+            t = _lib.RaggedTiles()
+            t.tile, t.stage_count, t.stage = edge, stage.shape[0], stage.data_ptr()
+            t.left_count, t.left = left.shape[0], left.data_ptr()
+            self._lists[edge] = (t, stage, left)
+        return self._lists[edge][0]
 
     @property
     def flops_per_step(self):
@@ -116,16 +179,24 @@ class RaggedLindblad:
         return 64.0 * self.work_units
 
     def step(self, dt, nsteps, stream=None):
-        """Advance every instance by ``nsteps`` RK4 steps: one kernel launch (async)."""
+        """Advance every instance by ``nsteps`` RK4 steps (async): one persistent launch
+        (``variant`` < ``variants()``), or one launch per phase of each stage."""
         from . import _lib
         r = _lib.RaggedBatch()
-        r.count, r.variant, r.max_groups = self.count, self.variant, self.max_groups
+        tiled = self.variant - self.variants()
+        r.count, r.max_groups = self.count, self.max_groups
         r.inst, r.order = self.inst.data_ptr(), self.order.data_ptr()
         r.ops, r.rho, r.work, r.queue = (self.ops.data_ptr(), self.rho.data_ptr(),
                                          self.work.data_ptr(), self.queue.data_ptr())
         p = _lib.StepParams()
         p.dt, p.nsteps = float(dt), int(nsteps)
         s = stream if stream is not None else torch.cuda.current_stream(self.dev)
+        if tiled >= 0:
+            tiles = self._tile_lists(TILE_EDGES[tiled])
+            _lib.check(self._lib.lime_lindblad_rk4_ragged_tiles(ctypes.byref(r), ctypes.byref(tiles),
+                                                                ctypes.byref(p), ctypes.c_void_p(s.cuda_stream)))
+            return
+        r.variant = self.variant
         _lib.check(self._lib.lime_lindblad_rk4_ragged(ctypes.byref(r), ctypes.byref(p),
                                                       ctypes.c_void_p(s.cuda_stream)))
 
