@@ -251,6 +251,25 @@ int lime_adjoint_contract_pairs(int32_t batch, int32_t n, int32_t pairs, const v
 int lime_adjoint_seed(int32_t batch, int32_t n, int32_t flags, void* lam, const void* g, const void* m,
                       double c, void* k4, void* k4_op, void* acc, void* stream);
 
+/*
+ * `nsteps` RK4 steps of the constant linear system dx/dt = G x for `rows` row vectors x of
+ * length m, in FP64 (complex128 everywhere): every state is stored.
+ *   g      [m][m]                 generator (row-major: dx_i/dt = sum_j G_ij x_j)
+ *   x      [rows][m]              states, updated in place
+ *   states [nsteps][rows][m]      the states after every step
+ *   eops   [n_e][m], obs [nsteps][rows][n_e]: obs = sum_j eops_ej x_j of every stored state,
+ *          or both NULL
+ *   work   lime_linear_rk4_workspace_bytes(m) bytes of device memory
+ * The step's increment is formed once (RK4 of a constant G is a polynomial of G) and steps are
+ * taken in blocks, so records differ from step-by-step RK4 by FP64 rounding.
+ * Replaces lime's _redfield (lime/oqs.py:373-472) and the loop of phys.expm (phys.py:1352-1401).
+ */
+int lime_linear_rk4(int32_t m, int32_t rows, int32_t nsteps, double dt, const void* g, void* x, void* states,
+                    int32_t n_e, const void* eops, void* obs, void* work, int64_t work_bytes, void* stream);
+
+/* Workspace bytes of lime_linear_rk4 for generators of dimension m. */
+int64_t lime_linear_rk4_workspace_bytes(int32_t m);
+
 /* Largest Hilbert dimension the resident (workspace-free) kernel accepts. */
 int lime_lindblad_max_n(int32_t n_dense, int32_t flags);
 

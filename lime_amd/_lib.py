@@ -37,6 +37,8 @@ EXPORTS = (
     "lime_adjoint_contract",
     "lime_adjoint_contract_pairs",
     "lime_adjoint_seed",
+    "lime_linear_rk4",
+    "lime_linear_rk4_workspace_bytes",
     "lime_last_error",
     "lime_version",
 )
@@ -177,6 +179,12 @@ def load(path=LIB_PATH):
         lib.lime_adjoint_seed.argtypes = [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, vp, vp, vp,
                                           ctypes.c_double, vp, vp, vp, vp]
         lib.lime_adjoint_seed.restype = ctypes.c_int
+        i32 = ctypes.c_int32
+        lib.lime_linear_rk4.argtypes = [i32, i32, i32, ctypes.c_double, vp, vp, vp, i32, vp, vp, vp,
+                                        ctypes.c_int64, vp]
+        lib.lime_linear_rk4.restype = ctypes.c_int
+        lib.lime_linear_rk4_workspace_bytes.argtypes = [i32]
+        lib.lime_linear_rk4_workspace_bytes.restype = ctypes.c_int64
         lib.lime_last_error.argtypes = []
         lib.lime_last_error.restype = ctypes.c_char_p
         lib.lime_version.argtypes = []

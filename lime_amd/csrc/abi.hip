@@ -8,6 +8,7 @@
 #include "lime_hip.h"
 #include "lindblad_resident_decl.hpp"
 #include "lindblad_tiled_decl.hpp"
+#include "linear_rk4_decl.hpp"
 
 static_assert(LIME_F_ONE_SIDED == lime::kFlagOneSided, "one flag value");
 static_assert(sizeof(lime_ragged_instance) == sizeof(lime::RaggedInstance) &&
@@ -325,6 +326,39 @@ int lime_lindblad_rk4_ragged_tiles(const lime_ragged_batch* r, const lime_ragged
   l.left = reinterpret_cast<const int2*>(t->left);
   hipError_t e = lime::ragged_tiles_run(a, l, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "lime_lindblad_rk4_ragged_tiles launch");
+  return LIME_OK;
+}
+
+int64_t lime_linear_rk4_workspace_bytes(int32_t m) {
+  return m < 1 ? 0 : (int64_t)lime::linear_workspace_bytes(m);
+}
+
+int lime_linear_rk4(int32_t m, int32_t rows, int32_t nsteps, double dt, const void* g, void* x, void* states,
+                    int32_t n_e, const void* eops, void* obs, void* work, int64_t work_bytes, void* stream) {
+  if (m < 1 || rows < 0 || nsteps < 0 || n_e < 0) return fail(LIME_ERR_ARG, "lime_linear_rk4: bad m, rows, nsteps or n_e");
+  if (rows == 0 || nsteps == 0) return LIME_OK;
+  if (!g || !x || !states) return fail(LIME_ERR_ARG, "lime_linear_rk4: g, x and states are required");
+  if ((eops == nullptr) != (obs == nullptr) || (obs != nullptr && n_e < 1))
+    return fail(LIME_ERR_ARG, "lime_linear_rk4: obs needs eops and n_e > 0");
+  if ((int64_t)nsteps * rows > INT32_MAX || (int64_t)lime::cdiv(m, 16) * lime::cdiv(m, 16) > INT32_MAX)
+    return fail(LIME_ERR_ARG, "lime_linear_rk4: nsteps * rows or m is too large");
+  const int64_t need = (int64_t)lime::linear_workspace_bytes(m);
+  if (work == nullptr || work_bytes < need)
+    return fail(LIME_ERR_ARG, "lime_linear_rk4: m = " + std::to_string(m) + " needs a workspace of " + std::to_string(need) +
+                                  " bytes (lime_linear_rk4_workspace_bytes)");
+  lime::LinearArgs a;
+  a.m = m;
+  a.rows = rows;
+  a.nsteps = nsteps;
+  a.n_e = n_e;
+  a.dt = dt;
+  a.gen = static_cast<const double2*>(g);
+  a.eops = static_cast<const double2*>(eops);
+  a.x = static_cast<double2*>(x);
+  a.states = static_cast<double2*>(states);
+  a.obs = static_cast<double2*>(obs);
+  hipError_t e = lime::linear_run(a, work, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "lime_linear_rk4 launch");
   return LIME_OK;
 }
 

@@ -104,8 +104,8 @@ def expm(A, t, method="EOM", precision="fp64"):
 
     'EOM': U(t_0) = I and each further entry one RK4 step of dU/dt = A U with
     dt = t[1] - t[0] (lime's ``interval``), i.e. U(t_k) = P(dt A)^k with the RK4 polynomial
-    P; the Nt - 1 steps run in one launch sequence of the one-sided per-stage kernels
-    (FP64 by default) recording every step.  'SOS' raises NotImplementedError, as in lime.
+    P; the Nt - 1 steps run on ``lime_linear_rk4`` in FP64 (the default), else on the
+    one-sided per-stage kernels, recording every step.  'SOS' raises NotImplementedError, as in lime.
     """
     if method == "SOS":
         raise NotImplementedError("Method of SOS has not been implemented. Choose from EOM")
@@ -113,9 +113,25 @@ def expm(A, t, method="EOM", precision="fp64"):
         raise ValueError(f"unknown method {method!r}")
     import torch
 
-    from .redfield import _column_chunk, liouville_propagator
+    from .redfield import _column_chunk, _dense, linear_rk4, liouville_propagator
     t = np.asarray(t, dtype=np.float64)
     Nt = len(t)
+    if precision == "fp64":
+        from .propagator import as_c128, device
+        At = as_c128(_dense(A), device())
+        if At.dim() != 2 or At.shape[0] != At.shape[1]:
+            raise ValueError(f"A must be (M, M), got {tuple(At.shape)}")
+        M = At.shape[0]
+        At = At.transpose(0, 1).contiguous()       # the rows of U step with A^T: U_k = U_(k-1) P(dt A)
+        x = torch.eye(M, dtype=torch.complex128, device=At.device)
+        out = [x.cpu().numpy()]
+        done, chunk = 1, _column_chunk(M)
+        while done < Nt:
+            m = min(chunk, Nt - done)
+            x, st, _ = linear_rk4(At, x, float(t[1] - t[0]), m)
+            out.extend(st.cpu().numpy())
+            done += m
+        return out
     prop = liouville_propagator(A, precision)
     M = prop.n
     U = torch.eye(M, dtype=torch.complex128, device=prop.dev).unsqueeze(0).contiguous()

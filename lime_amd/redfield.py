@@ -22,11 +22,14 @@ i.e. the Lindblad kernel's right-hand side with H_eff = G and 2K sandwich terms
 ``expect``/``correlation_2op_1t``/``correlation_4op_3t`` (oqs.py:145-366) evaluate the
 Liouville-space propagator U(t) on the GPU (eigendecomposition for 'SOS', RK4 for 'EOM').
 """
+import ctypes
+
 import numpy as np
 import scipy.sparse as sp
 import torch
 from scipy.linalg import eigh
 
+from . import _lib
 from . import superoperator as so
 from .mol import Result
 from .propagator import LindbladPropagator, as_c128, device
@@ -90,14 +93,75 @@ def _column_chunk(M, budget=1 << 28):
     return max(1, budget // (M * M * 16))
 
 
+def linear_rk4(G, x, dt, nsteps, eops=None, keep=True):
+    """``nsteps`` RK4 steps of dx/dt = G x (``lime_linear_rk4``, FP64) for the rows of ``x``
+    (rows, M), a complex128 tensor on the GPU.
+
+    Returns (the final rows, the rows after every step (nsteps, rows, M) or None without
+    ``keep``, sum_j eops[e, j] x_j after every step (nsteps, rows, n_e) or None)."""
+    dev = x.device
+    lib = _lib.load()
+    rows, M = x.shape
+    Gt = as_c128(G, dev)
+    if Gt.shape != (M, M):
+        raise ValueError(f"the generator has shape {tuple(Gt.shape)}, expected ({M}, {M})")
+    if eops is not None and tuple(eops.shape[1:]) != (M,):
+        raise ValueError(f"observables have shape {tuple(eops.shape)}, expected (n_e, {M})")
+    x = x.clone()
+    n_e = 0 if eops is None else eops.shape[0]
+    empty = lambda *shape: torch.empty(shape, dtype=torch.complex128, device=dev)
+    obs = empty(nsteps, rows, n_e) if n_e else None
+    # without `keep` the states of 256 MB of steps at a time are enough for the observables
+    chunk = nsteps if keep else max(1, min(nsteps, (1 << 28) // (rows * M * 16)))
+    states = empty(chunk, rows, M)
+    nbytes = int(lib.lime_linear_rk4_workspace_bytes(M))
+    work = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    ptr = lambda t: t.data_ptr() if t is not None else None
+    s = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    for done in range(0, nsteps, max(1, chunk)):
+        m = min(chunk, nsteps - done)
+        _lib.check(lib.lime_linear_rk4(M, rows, m, float(dt), Gt.data_ptr(), x.data_ptr(), states.data_ptr(), n_e,
+                                       ptr(eops), ptr(obs[done:done + m]) if obs is not None else None,
+                                       work.data_ptr(), nbytes, s))
+    return x, states if keep else None, obs
+
+
+def _redfield_columns(R, x0, dt, Nt, E, keep, precision):
+    """vec rho as column 0 of an M x M operator (other columns zero) on the one-sided kernels:
+    the reduced-precision form of ``_redfield``."""
+    dev, M = x0.device, x0.shape[0]
+    prop = liouville_propagator(R, precision)
+    X = torch.zeros((1, M, M), dtype=torch.complex128, device=dev)
+    X[0, :, 0] = x0
+    Et = None
+    if E is not None:
+        Et = torch.zeros((1, E.shape[0], M, M), dtype=torch.complex128, device=dev)
+        Et[0, :, :, 0] = E
+    obs = torch.zeros((1, Nt, E.shape[0]), dtype=torch.complex128, device=dev) if E is not None else None
+    cols = torch.empty((Nt, M), dtype=torch.complex128, device=dev) if keep else None
+    chunk = _column_chunk(M) if keep else Nt
+    done = 0
+    while done < Nt:
+        m = min(chunk, Nt - done)
+        # records at chunk-local indices 0..m-1 (one launch sequence per chunk)
+        st = torch.empty((1, m, M, M), dtype=torch.complex128, device=dev) if keep else None
+        ob = torch.empty((1, m, E.shape[0]), dtype=torch.complex128, device=dev) if E is not None else None
+        prop.step(X, dt, m, eops_t=Et, obs=ob, states=st, nout=1, step_offset=0, rec_capacity=m)
+        if ob is not None:
+            obs[:, done:done + m] = ob
+        if st is not None:
+            cols[done:done + m] = st[0, :, :, 0]
+        done += m
+    return X[0, :, 0], cols, obs[0] if obs is not None else None
+
+
 def _redfield(R, rho0, evecs=None, Nt=1, dt=0.005, t0=0, e_ops=None, return_result=True,
               precision="fp64"):
     """RK4 on vec rho with a dense Liouville tensor R (oqs.py:373-468 semantics).
 
-    vec rho is column 0 of an M x M operator X (M = N^2, other columns zero), stepped by
-    the one-sided kernels (dX/dt = R X) in launches of many steps; Tr[e rho] is the kernel's
-    record sum_m W_m0 X_m0 with W_m0 = e[m % N, m // N].  States are transformed back with
-    evecs (rho -> v rho v^dag), observables are taken in the eigenbasis, as lime does."""
+    FP64 (the default) steps vec rho by ``linear_rk4``; Tr[e rho] is sum_m W_m x_m with
+    W_m = e[m % N, m // N].  States are transformed back with evecs (rho -> v rho v^dag),
+    observables are taken in the eigenbasis, as lime does."""
     dev = device()
     e_ops = [] if e_ops is None else list(e_ops)
     r0 = _dense(rho0)
@@ -106,33 +170,19 @@ def _redfield(R, rho0, evecs=None, Nt=1, dt=0.005, t0=0, e_ops=None, return_resu
     if evecs is not None:
         r0 = evecs.conj().T @ r0 @ evecs
         e_ops = [evecs.conj().T @ _dense(e) @ evecs for e in e_ops]
-    prop = liouville_propagator(R, precision)
-    X = torch.zeros((1, M, M), dtype=torch.complex128, device=dev)
-    X[0, :, 0] = as_c128(r0.flatten(), dev)
-    Et = None
-    if e_ops:
-        Et = torch.zeros((1, len(e_ops), M, M), dtype=torch.complex128, device=dev)
-        for i, e in enumerate(e_ops):
-            Et[0, i, :, 0] = as_c128(_dense(e).T.flatten(), dev)     # e[m % N, m // N]
-    obs = torch.zeros((1, Nt, len(e_ops)), dtype=torch.complex128, device=dev) if e_ops else None
-    cols = torch.empty((Nt, M), dtype=torch.complex128, device=dev) if return_result else None
-    chunk = _column_chunk(M) if return_result else Nt
-    done = 0
-    while done < Nt:
-        m = min(chunk, Nt - done)
-        # records at chunk-local indices 0..m-1 (one launch sequence per chunk)
-        st = torch.empty((1, m, M, M), dtype=torch.complex128, device=dev) if return_result else None
-        ob = torch.empty((1, m, len(e_ops)), dtype=torch.complex128, device=dev) if e_ops else None
-        prop.step(X, dt, m, eops_t=Et, obs=ob, states=st, nout=1, step_offset=0, rec_capacity=m)
-        if ob is not None:
-            obs[:, done:done + m] = ob
-        if st is not None:
-            cols[done:done + m] = st[0, :, :, 0]
-        done += m
+    E = as_c128(np.stack([_dense(e).T.flatten() for e in e_ops]), dev) if e_ops else None   # e[m % N, m // N]
+    x0 = as_c128(r0.flatten(), dev)
+    if precision == "fp64":
+        x, cols, obs = linear_rk4(R, x0.reshape(1, M), dt, Nt, E, keep=return_result)
+        final = x[0]
+        cols = cols[:, 0] if cols is not None else None
+        obs = obs[:, 0] if obs is not None else None
+    else:
+        final, cols, obs = _redfield_columns(R, x0, dt, Nt, E, return_result, precision)
     if not return_result:
-        return _dense(X[0, :, 0].reshape(n, n))
+        return _dense(final.reshape(n, n))
     res = Result(dt=dt, Nt=Nt, rho0=rho0, t0=t0)
-    res.observables = _dense(obs[0]) if obs is not None else np.zeros((Nt, 0), np.complex128)
+    res.observables = _dense(obs) if obs is not None else np.zeros((Nt, 0), np.complex128)
     states = cols.reshape(Nt, n, n)
     if evecs is not None:
         V = as_c128(evecs, dev)
