@@ -113,6 +113,15 @@ typedef struct lime_step_params {
 int lime_lindblad_rk4(const lime_lindblad_batch* d, const lime_step_params* p, void* stream);
 
 /*
+ * lime_lindblad_rk4 with a generator per step (driven systems): d->heff is
+ * [nsteps][sets][n][n], step s of the call holds its H_eff over the four stages.  Everything
+ * else as in lime_lindblad_rk4, and the same bits as nsteps calls of one step.  FP32 at
+ * resident sizes runs all steps in one launch, other descriptors step by step.
+ * Replaces the time loop of lime's _lindblad_driven (lime/oqs.py:1691-1800).
+ */
+int lime_lindblad_rk4_driven(const lime_lindblad_batch* d, const lime_step_params* p, void* stream);
+
+/*
  * An uneven batch: `count` independent Lindblad systems of their own dimensions, packed.
  * Each instance's operators are complex64 regions of `ops` (H_eff, optional Hadamard
  * dissipator D, n_dense dense jump operators L_k, all n x n row-major), its state a

@@ -26,6 +26,7 @@ LIME_NOALLOC_SCRATCH_BYTES = 64 << 20
 #: every symbol include/lime_hip.h declares (checked by tests/test_abi.py)
 EXPORTS = (
     "lime_lindblad_rk4",
+    "lime_lindblad_rk4_driven",
     "lime_lindblad_rk4_noalloc",
     "lime_lindblad_rk4_ragged",
     "lime_lindblad_rk4_ragged_tiles",
@@ -146,6 +147,9 @@ def load(path=LIB_PATH):
         lib.lime_lindblad_rk4.argtypes = [ctypes.POINTER(LindbladBatch),
                                           ctypes.POINTER(StepParams), ctypes.c_void_p]
         lib.lime_lindblad_rk4.restype = ctypes.c_int
+        lib.lime_lindblad_rk4_driven.argtypes = [ctypes.POINTER(LindbladBatch),
+                                                 ctypes.POINTER(StepParams), ctypes.c_void_p]
+        lib.lime_lindblad_rk4_driven.restype = ctypes.c_int
         lib.lime_lindblad_rk4_noalloc.argtypes = [ctypes.POINTER(LindbladBatch),
                                                   ctypes.POINTER(StepParams), ctypes.c_void_p]
         lib.lime_lindblad_rk4_noalloc.restype = ctypes.c_int

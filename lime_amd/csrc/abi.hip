@@ -103,7 +103,7 @@ int scratch_for_current_device(void** out) {
 // lime_lindblad_rk4 with the per-stage workspace given explicitly (the caller's, or the
 // library's static scratch array for lime_lindblad_rk4_noalloc); `name` prefixes errors.
 int rk4_impl(const lime_lindblad_batch* d, const lime_step_params* p, void* stream, void* work,
-             int64_t work_bytes, const char* name, bool noalloc) {
+             int64_t work_bytes, const char* name, bool noalloc, bool driven = false) {
   if (d == nullptr || p == nullptr) return fail(LIME_ERR_ARG, std::string(name) + ": null descriptor");
   if (d->batch < 0 || d->n < 1) return fail(LIME_ERR_ARG, std::string(name) + ": batch must be >= 0 and n >= 1");
   if (d->batch == 0 || p->nsteps == 0) return LIME_OK;
@@ -121,6 +121,22 @@ int rk4_impl(const lime_lindblad_batch* d, const lime_step_params* p, void* stre
   if ((d->flags & LIME_F_PREC_MASK) == 0x30)
     return fail(LIME_ERR_UNSUPPORTED, std::string(name) + ": precision flag not built");
   const hipStream_t s = static_cast<hipStream_t>(stream);
+  // driven: one generator per step and set; the resident FP32 kernel (default shape) takes them
+  // all in one launch, the other paths go step by step
+  const int64_t heff_step = (int64_t)lime::cdiv(d->batch, d->group) * d->n * d->n;
+  if (driven && p->nsteps > 1 && (!use_resident(d) || use_resident_bf3(d) || resident_variant(d) != 0)) {
+    const int64_t bytes = heff_step * (is_fp64(d) ? sizeof(double2) : sizeof(float2));
+    for (int k = 0; k < p->nsteps; ++k) {
+      lime_lindblad_batch one = *d;
+      lime_step_params q = *p;
+      one.heff = static_cast<const unsigned char*>(d->heff) + k * bytes;
+      q.nsteps = 1;
+      q.step_offset = p->step_offset + k;
+      const int r = rk4_impl(&one, &q, stream, work, work_bytes, name, noalloc);
+      if (r != LIME_OK) return r;
+    }
+    return LIME_OK;
+  }
 
   if (use_resident(d)) {
     if (d->stage_states != nullptr)
@@ -147,6 +163,7 @@ int rk4_impl(const lime_lindblad_batch* d, const lime_step_params* p, void* stre
     a.nout = (d->obs || d->states) ? p->nout : 0;
     a.step_offset = p->step_offset;
     a.rec_capacity = p->rec_capacity;
+    a.heff_step = driven && p->nsteps > 1 ? heff_step : 0;
     hipError_t e = use_resident_bf3(d) ? lime::resident_bf3_launch(a, s) : lime::resident_launch(a, resident_variant(d), s);
     if (e != hipSuccess) return hip_fail(e, (std::string(name) + " (resident) launch").c_str());
     return LIME_OK;
@@ -228,6 +245,10 @@ int64_t lime_lindblad_workspace_bytes(const lime_lindblad_batch* d) {
 
 int lime_lindblad_rk4(const lime_lindblad_batch* d, const lime_step_params* p, void* stream) {
   return rk4_impl(d, p, stream, d ? d->work : nullptr, d ? d->work_bytes : 0, "lime_lindblad_rk4", false);
+}
+
+int lime_lindblad_rk4_driven(const lime_lindblad_batch* d, const lime_step_params* p, void* stream) {
+  return rk4_impl(d, p, stream, d ? d->work : nullptr, d ? d->work_bytes : 0, "lime_lindblad_rk4_driven", false, true);
 }
 
 int lime_lindblad_rk4_noalloc(const lime_lindblad_batch* d, const lime_step_params* p, void* stream) {

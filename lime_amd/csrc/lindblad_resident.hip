@@ -27,9 +27,14 @@ namespace lime {
 
 namespace {
 
-// D o S at one element (complex product d s)
+// spare elements after the resident dense operands (fragment prefetch past the last row)
+constexpr int kOpTail = 8;
+
+// D o S at one element (complex product d s).  The fused operations are written out: the compiler
+// fuses the plain expression one way before the step loop and another way in it, and a run cut
+// into several launches then differs from one launch in the last bit.
 __device__ __forceinline__ float2 cmulf(float2 d, float2 s) {
-  return make_float2(d.x * s.x - d.y * s.y, d.x * s.y + d.y * s.x);
+  return make_float2(fmaf(d.x, s.x, -(d.y * s.y)), fmaf(d.x, s.y, d.y * s.x));
 }
 
 // Copy a row-major n x n complex64 operator into an NP x P LDS buffer (zero padded).
@@ -46,17 +51,18 @@ __device__ __forceinline__ void stage_operator(float2* dst, const float2* __rest
 // Software-pipelined complex product over LDS operands for the wave's tiles:
 //   MODE 0: C += A B          (A rows from sA, B[k][j] = sB[k][j])
 //   MODE 2: C += i A M^dag    (A rows from sA, B[k][j] = conj(sM[j][k]), sM = sB)
-// The reduction runs over k < ke (operands are zero beyond n).  sA / sB may be read up to
-// 4 columns / rows past ke (padding, or the spare LDS after each buffer).
-template <int NP, int P, int BPW, int MODE>
-__device__ __forceinline__ void lds_gemm(const float2* sA, const float2* sB, const int (&trow)[BPW],
+// with row pitches PA and PB.  The reduction runs over k < ke (operands are zero beyond n).
+// sA / sB may be read up to 4 columns / rows past ke (padding, or the spare LDS after each
+// buffer).
+template <int BPW, int MODE>
+__device__ __forceinline__ void lds_gemm(const float2* sA, int PA, const float2* sB, int PB, const int (&trow)[BPW],
                                          const int (&tcol)[BPW], int lr, int lg, int ke, floatx4 (&cr)[BPW],
                                          floatx4 (&ci)[BPW]) {
   int oA[BPW], oB[BPW];
 #pragma unroll
   for (int u = 0; u < BPW; ++u) {
-    oA[u] = (trow[u] + lr) * P + lg;
-    oB[u] = (MODE == 0) ? lg * P + tcol[u] + lr : (tcol[u] + lr) * P + lg;
+    oA[u] = (trow[u] + lr) * PA + lg;
+    oB[u] = (MODE == 0) ? lg * PB + tcol[u] + lr : (tcol[u] + lr) * PB + lg;
   }
   float2 x[BPW], y[BPW];
 #pragma unroll
@@ -70,7 +76,7 @@ __device__ __forceinline__ void lds_gemm(const float2* sA, const float2* sB, con
 #pragma unroll
     for (int u = 0; u < BPW; ++u) {
       xn[u] = sA[oA[u] + k0 + 4];
-      yn[u] = sB[oB[u] + (MODE == 0 ? (k0 + 4) * P : k0 + 4)];
+      yn[u] = sB[oB[u] + (MODE == 0 ? (k0 + 4) * PB : k0 + 4)];
     }
 #pragma unroll
     for (int u = 0; u < BPW; ++u) {
@@ -95,6 +101,57 @@ __device__ __forceinline__ void lds_gemm(const float2* sA, const float2* sB, con
   }
 }
 
+// One loop over both: C += i T R^dag (into cr, ci; T and R^dag as MODE 2 of lds_gemm) and
+// U += L S (into tr, ti; MODE 0), each with lds_gemm's order of products.
+template <int BPW>
+__device__ __forceinline__ void lds_gemm_pair(const float2* sT, int PT, const float2* sR, const float2* sL, int PO,
+                                              const float2* sS, int PS, const int (&trow)[BPW], const int (&tcol)[BPW],
+                                              int lr, int lg, int ke, floatx4 (&cr)[BPW], floatx4 (&ci)[BPW],
+                                              floatx4 (&tr)[BPW], floatx4 (&ti)[BPW]) {
+  int oT[BPW], oR[BPW], oL[BPW], oS[BPW];
+  float2 x[BPW], y[BPW], z[BPW], h[BPW];
+#pragma unroll
+  for (int u = 0; u < BPW; ++u) {
+    oT[u] = (trow[u] + lr) * PT + lg;
+    oR[u] = (tcol[u] + lr) * PO + lg;
+    oL[u] = (trow[u] + lr) * PO + lg;
+    oS[u] = lg * PS + tcol[u] + lr;
+    x[u] = sT[oT[u]];
+    y[u] = sR[oR[u]];
+    z[u] = sL[oL[u]];
+    h[u] = sS[oS[u]];
+  }
+#pragma unroll 2
+  for (int k0 = 0; k0 < ke; k0 += 4) {
+    float2 xn[BPW], yn[BPW], zn[BPW], hn[BPW];
+#pragma unroll
+    for (int u = 0; u < BPW; ++u) {
+      xn[u] = sT[oT[u] + k0 + 4];
+      yn[u] = sR[oR[u] + k0 + 4];
+      zn[u] = sL[oL[u] + k0 + 4];
+      hn[u] = sS[oS[u] + (k0 + 4) * PS];
+    }
+#pragma unroll
+    for (int u = 0; u < BPW; ++u) {
+      cr[u] = mfma_f32(x[u].x, y[u].y, cr[u]);
+      ci[u] = mfma_f32(x[u].x, y[u].x, ci[u]);
+      tr[u] = mfma_f32(z[u].x, h[u].x, tr[u]);
+      ti[u] = mfma_f32(z[u].x, h[u].y, ti[u]);
+      cr[u] = mfma_f32(-x[u].y, y[u].x, cr[u]);
+      ci[u] = mfma_f32(x[u].y, y[u].y, ci[u]);
+      tr[u] = mfma_f32(-z[u].y, h[u].y, tr[u]);
+      ti[u] = mfma_f32(z[u].y, h[u].x, ti[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < BPW; ++u) {
+      x[u] = xn[u];
+      y[u] = yn[u];
+      z[u] = zn[u];
+      h[u] = hn[u];
+    }
+  }
+}
+
 }  // namespace
 
 // Bordered sizes (n = 16 m + 1, no dense jump operators): the last index is the border.
@@ -103,9 +160,14 @@ __device__ __forceinline__ void lds_gemm(const float2* sA, const float2* sB, con
 // border outputs (row 16m and column 16m) are 65-term-or-shorter complex dot products on
 // VALU, each split over BG lanes.  The padded size of the plain kernel would spend
 // (m+1)^2 tiles on these outputs instead of m^2.
-template <int NB, int W, int BPW, int MINW, bool DENSE, bool REC, bool BRD, bool DB>
-__global__ void __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(MINW)))
-lindblad_rk4_resident(ResidentArgs a) {
+//
+// DRV (driven systems): step s of the launch runs with the generator H_eff at a.heff + s
+// heff_step (elements), put into LDS between the steps; a launch per step reloaded every
+// operand, and cost a launch, for one step's work.
+// RES (dense jump operators): every L_k and R_k stays in LDS for the launch instead of being
+// staged through one buffer in each stage.
+template <int NB, int W, int BPW, int MINW, bool DENSE, bool REC, bool BRD, bool DB, bool DRV, bool RES>
+__device__ __forceinline__ void resident_body(const ResidentArgs& a) {
   // LDS rows / columns held: bordered layouts hold the core, the border index and 7 zero
   // ones (the reductions and the fragment prefetch read up to index 16 (NB - 1) + 7)
   constexpr int NP = BRD ? 16 * (NB - 1) + 8 : NB * 16;
@@ -152,8 +214,13 @@ lindblad_rk4_resident(ResidentArgs a) {
   // prefetch past the last k step
   float2* sS1 = DB ? sS0 + NP * P + 4 * P + 4 : sS0;
   float2* sT = sS1 + NP * P + 4 * P + 4;
-  float2* sL = sT + (DENSE ? NP * P + 4 * P + 4 : 0);
-  double2* sRed = reinterpret_cast<double2*>(sL + (DENSE ? NP * P + 4 * P + 4 : 0));
+  // dense operands: staged one after the other through sL, or (RES) all of them from sL on, NP
+  // rows of op_pitch elements each, with a second T buffer before them
+  const int slot = RES ? NP * a.op_pitch : 0;
+  float2* sT1 = sT + (RES ? NP * P + 4 * P + 4 : 0);
+  float2* sL = sT1 + (DENSE ? NP * P + 4 * P + 4 : 0);
+  double2* sRed = reinterpret_cast<double2*>(
+      sL + (RES ? a.n_dense * (a.rops ? 2 : 1) * slot + kOpTail : DENSE ? NP * P + 4 * P + 4 : 0));
 
   const int b = xcd_block();   // the operators of one generator set run on one XCD (shared L2)
   if (b >= a.batch) return;
@@ -181,6 +248,16 @@ lindblad_rk4_resident(ResidentArgs a) {
         sS0[i * P + j] = make_float2(0.f, 0.f);
         sS1[i * P + j] = make_float2(0.f, 0.f);
       }
+    }
+  }
+  if constexpr (RES) {
+    const int mats = a.n_dense * (a.rops ? 2 : 1);
+    for (int idx = tid; idx < mats * slot; idx += T) {
+      const int mat = idx / slot, e = idx - mat * slot;
+      const int i = e / a.op_pitch, j = e - i * a.op_pitch;
+      const float2* src = mat < a.n_dense ? a.lops + ((size_t)set * a.n_dense + mat) * nn
+                                          : a.rops + ((size_t)set * a.n_dense + mat - a.n_dense) * nn;
+      sL[idx] = i < n && j < n ? src[i * n + j] : make_float2(0.f, 0.f);
     }
   }
   if (BRD) __syncthreads();
@@ -505,9 +582,43 @@ lindblad_rk4_resident(ResidentArgs a) {
         br += dbr;
         bm += dbm;
       }
+      if constexpr (RES) {
+        // C += i sum_k (L_k S) R_k^dag, operands resident: the products T_k R_k^dag and
+        // L_k+1 S do not depend on each other and share one loop, T_k alternates between two
+        // buffers, so a term takes one loop and one barrier
+        floatx4 tr[BPW], ti[BPW];
+        const auto put_t = [&](float2* Tk) {
+#pragma unroll
+          for (int u = 0; u < BPW; ++u) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+              if (tval[u]) Tk[(trow[u] + 4 * lg + v) * P + tcol[u] + lr] = make_float2(tr[u][v], ti[u][v]);
+              tr[u][v] = 0.f;
+              ti[u][v] = 0.f;
+            }
+          }
+        };
+#pragma unroll
+        for (int u = 0; u < BPW; ++u) {
+          tr[u] = floatx4{0.f, 0.f, 0.f, 0.f};
+          ti[u] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+        lds_gemm<BPW, 0>(sL, a.op_pitch, sS, P, trow, tcol, lr, lg, ke, tr, ti);
+        put_t(sT);
+        __syncthreads();
+        const float2* R = sL + (a.rops ? a.n_dense * slot : 0);
+        int kk = 0;
+        for (; kk + 1 < a.n_dense; ++kk) {
+          lds_gemm_pair<BPW>(kk & 1 ? sT1 : sT, P, R + kk * slot, sL + (kk + 1) * slot, a.op_pitch, sS, P, trow, tcol, lr,
+                             lg, ke, cr, ci, tr, ti);
+          put_t(kk & 1 ? sT : sT1);
+          __syncthreads();
+        }
+        lds_gemm<BPW, 2>(kk & 1 ? sT1 : sT, P, R + kk * slot, a.op_pitch, trow, tcol, lr, lg, ke, cr, ci);
+      }
       // C += i sum_k (L_k S) R_k^dag, every factor staged through LDS (sL) so the fragment
       // loops are the same pipelined LDS reads as the H_eff products.
-      for (int kk = 0; DENSE && kk < a.n_dense; ++kk) {
+      for (int kk = 0; DENSE && !RES && kk < a.n_dense; ++kk) {
         const float2* L = a.lops + ((size_t)set * a.n_dense + kk) * nn;
         __syncthreads();                        // previous users of sL / sT are done
         stage_operator<NP, P, T>(sL, L, n, tid);
@@ -518,7 +629,7 @@ lindblad_rk4_resident(ResidentArgs a) {
           tr[u] = floatx4{0.f, 0.f, 0.f, 0.f};
           ti[u] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
-        lds_gemm<NP, P, BPW, 0>(sL, sS, trow, tcol, lr, lg, ke, tr, ti);    // T = L S
+        lds_gemm<BPW, 0>(sL, P, sS, P, trow, tcol, lr, lg, ke, tr, ti);    // T = L S
 #pragma unroll
         for (int u = 0; u < BPW; ++u) {
           if (!tval[u]) continue;
@@ -531,7 +642,7 @@ lindblad_rk4_resident(ResidentArgs a) {
           stage_operator<NP, P, T>(sL, a.rops + ((size_t)set * a.n_dense + kk) * nn, n, tid);
         }
         __syncthreads();
-        lds_gemm<NP, P, BPW, 2>(sT, sL, trow, tcol, lr, lg, ke, cr, ci);    // C += i T R^dag
+        lds_gemm<BPW, 2>(sT, P, sL, P, trow, tcol, lr, lg, ke, cr, ci);    // C += i T R^dag
       }
       // k = -i C + D o S, formed in place: afterwards kr = ci, ki = -cr.
       if (!DFOLD && has_d) {
@@ -740,6 +851,16 @@ lindblad_rk4_resident(ResidentArgs a) {
           if (BRD && bwrite) Sg[bi * n + bj] = rho_b;
         }
       }
+      if constexpr (DRV) {
+        if (s + 1 < a.nsteps) {
+          if (DB) __syncthreads();  // every wave has finished reading H_eff
+          const float2* H = a.heff + (size_t)(s + 1) * a.heff_step + (size_t)set * nn;
+          for (int idx = tid; idx < nn; idx += T) {
+            const int i = idx / n;
+            sH[i * P + idx - i * n] = H[idx];
+          }
+        }
+      }
       __syncthreads();  // S of the next step (and the record partials) are complete
       ph ^= (int)DB;
       // the record's final sums go to the last wave: in the bordered kernels it holds no
@@ -779,6 +900,25 @@ lindblad_rk4_resident(ResidentArgs a) {
   }
 }
 
+template <int NB, int W, int BPW, int MINW, bool DENSE, bool REC, bool BRD, bool DB>
+__global__ void __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(MINW)))
+lindblad_rk4_resident(ResidentArgs a) {
+  resident_body<NB, W, BPW, MINW, DENSE, REC, BRD, DB, false, false>(a);
+}
+
+// dense jump operators resident in LDS
+template <int NB, int W, int BPW, int MINW, bool REC>
+__global__ void __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(MINW)))
+lindblad_rk4_resident_ops(ResidentArgs a) {
+  resident_body<NB, W, BPW, MINW, true, REC, false, false, false, true>(a);
+}
+
+template <int NB, int W, int BPW, int MINW, bool DENSE, bool BRD, bool DB, bool RES>
+__global__ void __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(MINW)))
+lindblad_rk4_resident_driven(ResidentArgs a) {
+  resident_body<NB, W, BPW, MINW, DENSE, true, BRD, DB, true, RES>(a);
+}
+
 // ------------------------------------------------------------------------ host launch
 namespace {
 
@@ -809,21 +949,38 @@ constexpr Shape kBorderShapes[7][kMaxVariants] = {
     {},
 };
 
-template <int NB, int W, int BPW, int MINW, bool DENSE, bool REC, bool BRD, bool DB>
-hipError_t launch_one(const ResidentArgs& a, size_t lds, hipStream_t stream) {
-  auto k = lindblad_rk4_resident<NB, W, BPW, MINW, DENSE, REC, BRD, DB>;
+hipError_t launch_kernel(void (*k)(ResidentArgs), const ResidentArgs& a, int waves, size_t lds, hipStream_t stream) {
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k, dim3(a.batch), dim3(W * 64), lds, stream, a);
+  hipLaunchKernelGGL(k, dim3(a.batch), dim3(waves * 64), lds, stream, a);
   return hipGetLastError();
 }
 
 template <int NB, int W, int BPW, int MINW, bool DENSE, bool BRD, bool DB>
 hipError_t launch_rec2(const ResidentArgs& a, size_t lds, hipStream_t stream) {
   const bool rec = a.nout > 0 && (a.obs != nullptr || a.states != nullptr);
-  return rec ? launch_one<NB, W, BPW, MINW, DENSE, true, BRD, DB>(a, lds, stream)
-             : launch_one<NB, W, BPW, MINW, DENSE, false, BRD, DB>(a, lds, stream);
+  if (a.heff_step > 0) {
+    // driven systems run the default shape; at 6 waves per SIMD the step's extra addresses spill
+    // two registers, and the few operators of a driven call do not need the occupancy
+    constexpr Shape first = (BRD ? kBorderShapes : kShapes)[NB][0];
+    constexpr int MW = MINW > 5 ? 5 : MINW;
+    if constexpr (W == first.w && BPW == first.bpw) {
+      if constexpr (DENSE && BPW == 1) {
+        if (a.op_pitch > 0)
+          return launch_kernel(lindblad_rk4_resident_driven<NB, W, BPW, MW, DENSE, BRD, DB, true>, a, W, lds, stream);
+      }
+      return launch_kernel(lindblad_rk4_resident_driven<NB, W, BPW, MW, DENSE, BRD, DB, false>, a, W, lds, stream);
+    }
+    return hipErrorInvalidValue;
+  }
+  if constexpr (DENSE && BPW == 1) {
+    if (a.op_pitch > 0)
+      return rec ? launch_kernel(lindblad_rk4_resident_ops<NB, W, BPW, MINW, true>, a, W, lds, stream)
+                 : launch_kernel(lindblad_rk4_resident_ops<NB, W, BPW, MINW, false>, a, W, lds, stream);
+  }
+  return rec ? launch_kernel(lindblad_rk4_resident<NB, W, BPW, MINW, DENSE, true, BRD, DB>, a, W, lds, stream)
+             : launch_kernel(lindblad_rk4_resident<NB, W, BPW, MINW, DENSE, false, BRD, DB>, a, W, lds, stream);
 }
 
 template <int NB, int W, int BPW, int MINW, bool DENSE, bool BRD>
@@ -866,6 +1023,25 @@ const Shape& shape_of(int nb, int variant, bool brd) {
 }
 
 constexpr size_t kLdsMax = 160 * 1024;
+constexpr int kCUs = 256;
+size_t lds_layout(int n, int variant, int n_dense, int n_eops, int nbuf);
+
+// All dense operands resident in LDS: pitch of their rows (odd, the reduction length rounded up),
+// or 0 to stage them.  They are resident when the workgroups that the batch puts on a CU still
+// fit with them, so the occupancy of a large batch is never given up; shapes with one tile per
+// wave only (with two the shared loop spills).  us per RK4 step, staged / resident, one operator:
+// n = 8, 16 jump operators 56.6 / 35.9; n = 24, 4 sandwich terms 44 / 26, 16 jump operators 127 /
+// 85; n = 32, 4 45 / 33; n = 48, 4 120 / 106; n = 64, 1 75.4 / 74.9; 256 operators n = 32, 4 48 / 37.
+// The second T buffer takes the place of the staging buffer of the staged layout.
+int operand_pitch(int n) { return ((n + 3) & ~3) + 1; }
+size_t dense_lds_bytes(int n, int n_dense, bool rops) {
+  return ((size_t)n_dense * (rops ? 2 : 1) * 16 * cdiv(n, 16) * operand_pitch(n) + kOpTail) * sizeof(float2);
+}
+int dense_pitch(int n, int variant, int n_dense, int n_eops, bool rops, int batch) {
+  if (shape_of(cdiv(n, 16), variant, false).bpw != 1) return 0;
+  const size_t bytes = lds_layout(n, variant, n_dense, n_eops, 3) + dense_lds_bytes(n, n_dense, rops);
+  return bytes * cdiv(batch, kCUs) <= kLdsMax ? operand_pitch(n) : 0;
+}
 
 // LDS bytes of the layout: H_eff + nbuf operator buffers (NP x (NP+1) complex64 plus the
 // prefetch spare rows) + the FP64 reduction slots
@@ -907,9 +1083,14 @@ bool resident_double_buffered(int n, int variant, int n_dense, int n_eops) {
   return n_dense == 0 && cdiv(n, 16) <= 5 && lds_layout(n, variant, n_dense, n_eops, 2) <= kLdsMax;
 }
 
-hipError_t resident_launch(const ResidentArgs& a, int variant, hipStream_t stream) {
+hipError_t resident_launch(const ResidentArgs& args, int variant, hipStream_t stream) {
+  ResidentArgs a = args;
   if (variant < 0 || variant >= resident_variants(a.n, a.n_dense)) return hipErrorInvalidValue;
-  const size_t lds = resident_lds_bytes(a.n, variant, a.n_dense, a.n_eops);
+  size_t lds = resident_lds_bytes(a.n, variant, a.n_dense, a.n_eops);
+  if (a.n_dense > 0) {
+    a.op_pitch = dense_pitch(a.n, variant, a.n_dense, a.n_eops, a.rops != nullptr, a.batch);
+    if (a.op_pitch > 0) lds += dense_lds_bytes(a.n, a.n_dense, a.rops != nullptr);
+  }
   const bool db = resident_double_buffered(a.n, variant, a.n_dense, a.n_eops);
   const int nb = cdiv(a.n, 16);
   if (resident_bordered(a.n, a.n_dense)) {

@@ -18,6 +18,8 @@ struct ResidentArgs {
   double2* states;
   double dt;
   int nsteps, nout, step_offset, rec_capacity;
+  long long heff_step = 0;   // > 0: step s runs with H_eff at heff + s heff_step (driven systems)
+  int op_pitch = 0;          // set by resident_launch: row pitch of LDS-resident dense operands
 };
 
 int resident_nb_max(int n_dense);

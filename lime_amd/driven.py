@@ -6,10 +6,10 @@ for Hermitian H) and H(t) = H0 - sum_i f_i(t) H_i is evaluated at the END of eac
 lime.  lime builds H(t) with ``Ht = H[0]; Ht += ...`` which aliases and mutates the caller's
 H0 on every step (oqs.py:1717-1724); here H(t) is built fresh and H0 is never modified.
 
-Each step is one launch of the fused kernel with H_eff(t) (jump operators are folded once):
-the drive coefficients f_i(t_k) are evaluated on the host up front, and the H_eff(t_k) of a
-chunk of steps are formed on the GPU in one product, so a step launches nothing but the
-propagation; observables and states are recorded after every step.
+The jump operators are folded once, the drive coefficients f_i(t_k) evaluated on the host up
+front, and the H_eff(t_k) of a chunk of steps formed on the GPU in one product; the chunk's
+steps then run in one call (``lime_lindblad_rk4_driven``: at resident sizes one launch);
+observables and states are recorded after every step.
 """
 import numpy as np
 import torch
@@ -42,16 +42,14 @@ def _lindblad_driven(H, rho0, c_ops=None, e_ops=None, Nt=1, dt=0.005, t0=0.0,
             coef[k, i] = complex(f(t))
     Hd = torch.stack([h for h, _ in drives]).reshape(len(drives), n * n) if drives else None
     chunk = max(1, min(Nt, (64 << 20) // (16 * n * n)))   # H_eff(t) of up to 64 MiB of steps
+    heff_t = None
     for c0 in range(0, Nt, chunk):
         c1 = min(Nt, c0 + chunk)
         if Hd is not None:
             cf = torch.as_tensor(coef[c0:c1], device=dev)
-            heff_t = (heff0.reshape(1, n * n) - cf @ Hd).reshape(c1 - c0, n, n).to(prop.heff.dtype)
-        for k in range(c0, c1):
-            if Hd is not None:
-                prop.heff = heff_t[k - c0]
-            prop.step(rho, dt, 1, eops_t=E_t, eop_group=1, obs=obs, states=states, nout=1,
-                      step_offset=k, rec_capacity=Nt)
+            heff_t = (heff0.reshape(1, n * n) - cf @ Hd).reshape(c1 - c0, 1, n, n).to(prop.heff.dtype)
+        prop.step(rho, dt, c1 - c0, eops_t=E_t, eop_group=1, obs=obs, states=states, nout=1,
+                  step_offset=c0, rec_capacity=Nt, heff_steps=heff_t)
     if not return_result:
         # lime's files (oqs.py:1743-1773): obs.dat with the accumulated time column, and an
         # empty den_mat.dat that lime opens and closes without writing

@@ -291,13 +291,18 @@ class LindbladPropagator:
         return self._lib.lime_lindblad_max_n(self.n_dense, _PREC_FLAGS[self.precision])
 
     def step(self, rho, dt, nsteps, *, eops_t=None, eop_group=None, obs=None, states=None,
-             nout=1, step_offset=0, rec_capacity=0, renorm=False, stream=None, stage_states=None):
+             nout=1, step_offset=0, rec_capacity=0, renorm=False, stream=None, stage_states=None,
+             heff_steps=None):
         """Advance ``rho`` (B, N, N) complex128 in place by ``nsteps`` RK4 steps (async).
 
         ``stage_states`` (rec_capacity, 3, B, N, N) complex128 (record-major) receives the
         FP64 stage operands X + h/2 k1, X + h/2 k2, X + h k3 of every recorded step
-        (per-stage kernels: the propagator must be ``force_tiled`` for n <= 80)."""
+        (per-stage kernels: the propagator must be ``force_tiled`` for n <= 80).
+        ``heff_steps`` (nsteps, nsets, N, N) in the operand precision: the effective
+        Hamiltonian of every step (driven systems) in the place of the propagator's own."""
         n, B = self.n, self.batch
+        if heff_steps is not None:
+            _check(heff_steps, "heff_steps", (int(nsteps), self.nsets, n, n), self.operand_dtype, self.dev)
         _check(rho, "rho", (B, n, n), torch.complex128, self.dev)
         eop_group = int(eop_group or B)
         if eop_group < 1:
@@ -342,8 +347,10 @@ class LindbladPropagator:
         p.dt, p.nsteps, p.nout = float(dt), int(nsteps), int(nout)
         p.step_offset, p.rec_capacity = int(step_offset), int(rec_capacity)
         s = stream if stream is not None else torch.cuda.current_stream(self.dev)
-        _lib.check(self._lib.lime_lindblad_rk4(ctypes.byref(d), ctypes.byref(p),
-                                               ctypes.c_void_p(s.cuda_stream)))
+        if heff_steps is not None:
+            d.heff = heff_steps.data_ptr()
+        call = self._lib.lime_lindblad_rk4 if heff_steps is None else self._lib.lime_lindblad_rk4_driven
+        _lib.check(call(ctypes.byref(d), ctypes.byref(p), ctypes.c_void_p(s.cuda_stream)))
 
     def run(self, rho0, dt, nsteps, e_ops=None, nout=1, store_states=False, renorm=False,
             eop_group=None, chunk=None):
