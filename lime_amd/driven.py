@@ -16,7 +16,7 @@ import torch
 
 from . import datfile
 from .mol import Result
-from .propagator import LindbladPropagator, as_c128, device
+from .propagator import LindbladPropagator, as_c128, as_c128_stack, device
 
 
 def _lindblad_driven(H, rho0, c_ops=None, e_ops=None, Nt=1, dt=0.005, t0=0.0,
@@ -29,7 +29,7 @@ def _lindblad_driven(H, rho0, c_ops=None, e_ops=None, Nt=1, dt=0.005, t0=0.0,
     heff0 = prop.heff_c128                              # H0 - (i/2) sum L^dag L, complex128
     n = prop.n
     rho = as_c128(rho0, dev).reshape(1, n, n).clone()
-    E_t = torch.stack([as_c128(e, dev) for e in e_ops]).unsqueeze(0).transpose(-1, -2).contiguous() \
+    E_t = as_c128_stack(e_ops, dev).unsqueeze(0).transpose(-1, -2).contiguous() \
         if e_ops else None
     obs = torch.zeros((1, Nt, len(e_ops)), dtype=torch.complex128, device=dev) if e_ops else None
     states = torch.empty((1, Nt, n, n), dtype=torch.complex128, device=dev) if return_result else None

@@ -211,6 +211,14 @@ class Lindblad_solver:
         """
         dev = device()
         a_op, b_op, c_op = [as_c128(o, dev) for o in ops]
+        H = as_c128(self.H, dev)
+        r0 = as_c128(rho0, dev)
+        if H.dim() == 2 and r0.dim() == 2 and Nt > 0:          # one fold of the operators for both runs
+            prop = LindbladPropagator(H, self.c_ops or [], precision=self.precision)
+            _, _, states = prop.run(r0, dt, Nt, store_states=True)
+            X = torch.matmul(torch.matmul(c_op, states[0]), a_op).contiguous()     # (Nt, N, N)
+            _, obs, _ = prop.regrouped(Nt).run(X, dt, Ntau, e_ops=[b_op])
+            return _np(obs)[:, :, 0]
         _, _, states = _run(self.H, rho0, self.c_ops, dt, Nt, None, store_states=True,
                             precision=self.precision)
         X = torch.matmul(torch.matmul(c_op, states[0]), a_op).contiguous()     # (Nt, N, N)
