@@ -66,7 +66,7 @@ bool use_resident(const lime_lindblad_batch* d) {
 int tiled_tile(const lime_lindblad_batch* d) {
   if (d->variant == 1 || d->variant == 3 || d->variant == 4) return 32;
   if (d->variant == 2) return 64;
-  return lime::tiled_pick(d->batch, d->n);
+  return lime::tiled_pick(d->batch, d->n, d->n_dense, is_split_bf16(d));
 }
 int tiled_ksplit(const lime_lindblad_batch* d) { return d->variant == 3 ? 2 : d->variant == 4 ? 8 : 1; }
 

@@ -57,73 +57,72 @@ template <> struct CT<double> {
 //   I_AH  : C += i A M^dag
 enum Mode { PLAIN = 0, NEG_AH = 1, I_AH = 2 };
 
-// Load a TILE x PW panel of a row-major n x n matrix: rows r0.., cols k0..
-template <int TILE, int PW, typename C, bool FAST = false>
-__device__ __forceinline__ void load_rows(const C* __restrict__ M, int n, int r0, int k0,
-                                          C (&reg)[TILE * PW / 256], int tid) {
-  if (FAST && r0 + TILE <= n && k0 + PW <= n) {   // interior panel (uniform): no bounds tests
+// A panel of a row-major n x n matrix on its way to LDS: TILE rows x KW columns (the k index along
+// the columns, ROWS) or KW rows x TILE columns (k along the rows).  The element offsets of a thread
+// are formed once per product; a panel is then loads at one wave-uniform address plus those
+// 32-bit offsets, so a whole panel costs no vector instruction but its loads.  (Rows and columns
+// beyond the operator read the last valid one: they only reach outputs that are not stored.)
+// Bounds tests and 64-bit addresses per element took 28 of the 40 vector instructions of a panel of
+// the 32-tiles, and matrix and vector work overlap little (64 x n = 256, FP32: 54 % MFMA and 30 %
+// VALU busy).  us per RK4 step with them / without, 32-tiles: 64 x n = 256 602 / 551, 256 x n = 129
+// 464 / 415, FP64 64 x n = 256 1077 / 978; 64-tiles: 16 x n = 512 with 16 jump operators 15910 / 14360.
+template <int TILE, bool ROWS, typename C>
+struct Panel {
+  static constexpr int NR = TILE * KW / 256;
+  const char* base;              // wave-uniform: the panel's first element
+  unsigned step;                 // bytes from panel to panel
+  unsigned off[NR];
+  C reg[NR];
+  // first: first row (ROWS) or column of the tile; kb: first k
+  __device__ __forceinline__ void init(const C* M, int n, int first, int kb, int tid) {
+    const int f = first < n ? first : n - 1;
+    base = reinterpret_cast<const char*>(ROWS ? M + (size_t)f * n + kb : M + (size_t)kb * n + f);
+    step = (ROWS ? KW : KW * (unsigned)n) * (unsigned)sizeof(C);
 #pragma unroll
-    for (int q = 0; q < TILE * PW / 256; ++q) {
+    for (int q = 0; q < NR; ++q) {
       const int e = tid + q * 256;
-      reg[q] = M[(size_t)(r0 + e / PW) * n + k0 + e % PW];
+      const int r = ROWS ? e / KW : e / TILE, c = ROWS ? e % KW : e % TILE;
+      const int x = first + (ROWS ? r : c), g = (x < n ? x : n - 1) - f;
+      off[q] = (unsigned)(ROWS ? g * n + c : r * n + g) * (unsigned)sizeof(C);
     }
-    return;
   }
-#pragma unroll
-  for (int q = 0; q < TILE * PW / 256; ++q) {
+  // k of the thread's element q within the panel
+  static __device__ __forceinline__ int k_of(int q, int tid) {
     const int e = tid + q * 256;
-    const int r = e / PW, c = e % PW;
-    const int gr = r0 + r, gc = k0 + c;
-    C v;
-    v.x = 0;
-    v.y = 0;
-    if (gr < n && gc < n) v = M[(size_t)gr * n + gc];
-    reg[q] = v;
+    return ROWS ? e % KW : e / TILE;
   }
-}
-
-template <int TILE, int PW, typename C>
-__device__ __forceinline__ void store_rows(C* sM, const C (&reg)[TILE * PW / 256], int tid) {
+  // Load the next panel, of which `left` values of k lie in the operator.  The loads are the same
+  // instructions either way (a branch around them would wait for the data where it ends); the
+  // last panel's addresses stop at its last value of k and store() puts zeros beyond it.
+  __device__ __forceinline__ void load(int n, int left, int tid) {
+    if (left < KW) {
 #pragma unroll
-  for (int q = 0; q < TILE * PW / 256; ++q) {
-    const int e = tid + q * 256;
-    sM[(e / PW) * (PW + 1) + e % PW] = reg[q];
+      for (int q = 0; q < NR; ++q) {
+        const int over = k_of(q, tid) - (left - 1);
+        if (over > 0) off[q] -= (unsigned)((ROWS ? 1 : n) * over) * (unsigned)sizeof(C);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < NR; ++q) reg[q] = *reinterpret_cast<const C*>(base + off[q]);
+    base += step;
   }
-}
-
-// Load a PW x TILE panel: rows k0.. (the k index), cols c0..
-template <int TILE, int PW, typename C, bool FAST = false>
-__device__ __forceinline__ void load_cols(const C* __restrict__ M, int n, int k0, int c0,
-                                          C (&reg)[TILE * PW / 256], int tid) {
-  if (FAST && k0 + PW <= n && c0 + TILE <= n) {   // interior panel (uniform): no bounds tests
+  __device__ __forceinline__ void store(C* sM, int left, int tid) {
+    if (left < KW) {
 #pragma unroll
-    for (int q = 0; q < TILE * PW / 256; ++q) {
+      for (int q = 0; q < NR; ++q)
+        if (k_of(q, tid) >= left) {
+          reg[q].x = 0;
+          reg[q].y = 0;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
       const int e = tid + q * 256;
-      reg[q] = M[(size_t)(k0 + e / TILE) * n + c0 + e % TILE];
+      if (ROWS) sM[(e / KW) * KWP + e % KW] = reg[q];
+      else sM[(e / TILE) * (TILE + 1) + e % TILE] = reg[q];
     }
-    return;
   }
-#pragma unroll
-  for (int q = 0; q < TILE * PW / 256; ++q) {
-    const int e = tid + q * 256;
-    const int r = e / TILE, c = e % TILE;
-    const int gr = k0 + r, gc = c0 + c;
-    C v;
-    v.x = 0;
-    v.y = 0;
-    if (gr < n && gc < n) v = M[(size_t)gr * n + gc];
-    reg[q] = v;
-  }
-}
-
-template <int TILE, int PW, typename C>
-__device__ __forceinline__ void store_cols(C* sM, const C (&reg)[TILE * PW / 256], int tid) {
-#pragma unroll
-  for (int q = 0; q < TILE * PW / 256; ++q) {
-    const int e = tid + q * 256;
-    sM[(e / TILE) * (TILE + 1) + e % TILE] = reg[q];
-  }
-}
+};
 
 template <int TILE>
 constexpr int smem_b() { return KW * (TILE + 1) > TILE * KWP ? KW * (TILE + 1) : TILE * KWP; }
@@ -135,7 +134,7 @@ constexpr int smem_b() { return KW * (TILE + 1) > TILE * KWP ? KW * (TILE + 1) :
 //   PLAIN  (C += a h)         R1 += ax hx,   R2 += ay hy,  M1 += (ax + ay)(hx + hy)
 //   NEG_AH (C -= a conj(h))   R1 += -ax hx,  R2 += ay hy,  M1 += (ax + ay)(hy - hx)
 //   I_AH   (C += i a conj(h)) R1 += ax hy,   R2 += ay hx,  M1 += (ax + ay)(hx + hy)
-template <int TILE, int MODE, typename R, bool FAST = false>
+template <int TILE, int MODE, typename R>
 __device__ __forceinline__ void gemm_term(const typename CT<R>::C* __restrict__ A,
                                           const typename CT<R>::C* __restrict__ Bsrc, int n, int row0,
                                           int col0, typename CT<R>::C* sA, typename CT<R>::C* sB,
@@ -145,7 +144,6 @@ __device__ __forceinline__ void gemm_term(const typename CT<R>::C* __restrict__ 
                                           int wc, int lr, int lg, int kb, int ke) {
   using C = typename CT<R>::C;
   constexpr int BW = TILE / 32;
-  constexpr int NR = TILE * KW / 256;
   // 16x16 blocks entirely outside the operator hold zeros: their MFMAs are skipped
   // (wave-uniform), which frees the matrix pipe for the other workgroups of the CU
   bool rlive[BW], clive[BW];
@@ -154,55 +152,276 @@ __device__ __forceinline__ void gemm_term(const typename CT<R>::C* __restrict__ 
     rlive[p] = row0 + wr * (TILE / 2) + p * 16 < n;
     clive[p] = col0 + wc * (TILE / 2) + p * 16 < n;
   }
+  bool all_live = true;
+#pragma unroll
+  for (int p = 0; p < BW; ++p) all_live = all_live && rlive[p] && clive[p];
   // the reduction runs over k in [kb, ke): kb a multiple of the panel width, ke = n or a
-  // multiple of it (a K-split part), so no panel straddles two parts
-  C ra[NR], rb[NR];
-  load_rows<TILE, KW, C, FAST>(A, n, row0, kb, ra, tid);
-  if (MODE == PLAIN) load_cols<TILE, KW, C, FAST>(Bsrc, n, kb, col0, rb, tid);
-  else load_rows<TILE, KW, C, FAST>(Bsrc, n, col0, kb, rb, tid);
-  for (int k0 = kb; k0 < ke; k0 += KW) {
+  // multiple of it (a K-split part), so no panel straddles two parts.  kb < ke: a panel's loads are not
+  // tested against n
+  Panel<TILE, true, C> pa;
+  Panel<TILE, MODE != PLAIN, C> pb;
+  pa.init(A, n, row0, kb, tid);
+  pb.init(Bsrc, n, col0, kb, tid);
+  pa.load(n, n - kb, tid);
+  pb.load(n, n - kb, tid);
+  const auto stage = [&](int k0) {
     __syncthreads();                          // previous panel fully consumed
-    store_rows<TILE, KW>(sA, ra, tid);
-    if (MODE == PLAIN) store_cols<TILE, KW>(sB, rb, tid);
-    else store_rows<TILE, KW>(sB, rb, tid);
+    pa.store(sA, n - k0, tid);
+    pb.store(sB, n - k0, tid);
     __syncthreads();
     if (k0 + KW < ke) {                       // prefetch the next panel into registers
-      load_rows<TILE, KW, C, FAST>(A, n, row0, k0 + KW, ra, tid);
-      if (MODE == PLAIN) load_cols<TILE, KW, C, FAST>(Bsrc, n, k0 + KW, col0, rb, tid);
-      else load_rows<TILE, KW, C, FAST>(Bsrc, n, col0, k0 + KW, rb, tid);
+      pa.load(n, n - k0 - KW, tid);
+      pb.load(n, n - k0 - KW, tid);
     }
+  };
+  const auto frag_a = [&](int kk, int p) { return sA[(wr * (TILE / 2) + p * 16 + lr) * KWP + kk + lg]; };
+  const auto frag_b = [&](int kk, int p) {
+    return MODE == PLAIN ? sB[(kk + lg) * (TILE + 1) + wc * (TILE / 2) + p * 16 + lr]
+                         : sB[(wc * (TILE / 2) + p * 16 + lr) * KWP + kk + lg];
+  };
+  const auto product = [&](const C a, const C h, int p, int q) {
+    const R as = a.x + a.y;
+    if (MODE == PLAIN) {
+      cr[p][q] = CT<R>::mfma(a.x, h.x, cr[p][q]);
+      dr[p][q] = CT<R>::mfma(a.y, h.y, dr[p][q]);
+      ci[p][q] = CT<R>::mfma(as, h.x + h.y, ci[p][q]);
+    } else if (MODE == NEG_AH) {
+      cr[p][q] = CT<R>::mfma(-a.x, h.x, cr[p][q]);
+      dr[p][q] = CT<R>::mfma(a.y, h.y, dr[p][q]);
+      ci[p][q] = CT<R>::mfma(as, h.y - h.x, ci[p][q]);
+    } else {
+      cr[p][q] = CT<R>::mfma(a.x, h.y, cr[p][q]);
+      dr[p][q] = CT<R>::mfma(a.y, h.x, dr[p][q]);
+      ci[p][q] = CT<R>::mfma(as, h.x + h.y, ci[p][q]);
+    }
+  };
+  int k0 = kb;
+  // whole panels of blocks inside the operator: one basic block a panel, its fragment reads ahead
+  // of the products (a test per k-step left every read's latency in front of its three MFMAs).  A
+  // loop of its own: a branch inside one loop makes the compiler keep two sets of accumulators and
+  // copy between them.  FP64 keeps one loop: the fragments' registers cost it waves.  us per RK4
+  // step, FP32, tested / here: 16 x n = 512 with 16 jump operators (64-tiles) 14360 / 13630, one of
+  // them (32) 1686 / 1519, 16 x n = 256 with 4 (32) 732 / 681, 16 x n = 129 69 / 65.
+  if (sizeof(R) == 4 && all_live) {
+    for (; k0 < ke && k0 + KW <= n; k0 += KW) {
+      stage(k0);
+      C x[KW / 4][BW], y[KW / 4][BW];
 #pragma unroll
-    for (int kk = 0; kk < KW; kk += 4) {
-      if (k0 + kk >= n) break;                // the last panel: k-steps past n are zeros
-      C x[BW], y[BW];
+      for (int kk = 0; kk < KW / 4; ++kk)
 #pragma unroll
-      for (int p = 0; p < BW; ++p) {
-        x[p] = sA[(wr * (TILE / 2) + p * 16 + lr) * KWP + kk + lg];
-        if (MODE == PLAIN) y[p] = sB[(kk + lg) * (TILE + 1) + wc * (TILE / 2) + p * 16 + lr];
-        else y[p] = sB[(wc * (TILE / 2) + p * 16 + lr) * KWP + kk + lg];
-      }
-#pragma unroll
-      for (int p = 0; p < BW; ++p)
-#pragma unroll
-        for (int q = 0; q < BW; ++q) {
-          if (!(rlive[p] && clive[q])) continue;
-          const C a = x[p], h = y[q];
-          const R as = a.x + a.y;
-          if (MODE == PLAIN) {
-            cr[p][q] = CT<R>::mfma(a.x, h.x, cr[p][q]);
-            dr[p][q] = CT<R>::mfma(a.y, h.y, dr[p][q]);
-            ci[p][q] = CT<R>::mfma(as, h.x + h.y, ci[p][q]);
-          } else if (MODE == NEG_AH) {
-            cr[p][q] = CT<R>::mfma(-a.x, h.x, cr[p][q]);
-            dr[p][q] = CT<R>::mfma(a.y, h.y, dr[p][q]);
-            ci[p][q] = CT<R>::mfma(as, h.y - h.x, ci[p][q]);
-          } else {
-            cr[p][q] = CT<R>::mfma(a.x, h.y, cr[p][q]);
-            dr[p][q] = CT<R>::mfma(a.y, h.x, dr[p][q]);
-            ci[p][q] = CT<R>::mfma(as, h.x + h.y, ci[p][q]);
-          }
+        for (int p = 0; p < BW; ++p) {
+          x[kk][p] = frag_a(4 * kk, p);
+          y[kk][p] = frag_b(4 * kk, p);
         }
+#pragma unroll
+      for (int kk = 0; kk < KW / 4; ++kk)
+#pragma unroll
+        for (int p = 0; p < BW; ++p)
+#pragma unroll
+          for (int q = 0; q < BW; ++q) product(x[kk][p], y[kk][q], p, q);
     }
+  }
+  const auto k_step = [&](int kk) {
+    C x[BW], y[BW];
+#pragma unroll
+    for (int p = 0; p < BW; ++p) {
+      x[p] = frag_a(kk, p);
+      y[p] = frag_b(kk, p);
+    }
+#pragma unroll
+    for (int p = 0; p < BW; ++p)
+#pragma unroll
+      for (int q = 0; q < BW; ++q)
+        if (rlive[p] && clive[q]) product(x[p], y[q], p, q);
+  };
+  if constexpr (sizeof(R) == 4) {             // few panels come here: kept small
+    for (; k0 < ke; k0 += KW) {
+      stage(k0);
+#pragma unroll 1
+      for (int kk = 0; kk < KW && k0 + kk < n; kk += 4) k_step(kk);   // k-steps past n are zeros
+    }
+  } else {
+    for (; k0 < ke; k0 += KW) {
+      stage(k0);
+#pragma unroll
+      for (int kk = 0; kk < KW; kk += 4) {
+        if (k0 + kk >= n) break;
+        C x[BW], y[BW];
+#pragma unroll
+        for (int p = 0; p < BW; ++p) {
+          x[p] = frag_a(kk, p);
+          y[p] = frag_b(kk, p);
+        }
+#pragma unroll
+        for (int p = 0; p < BW; ++p)
+#pragma unroll
+          for (int q = 0; q < BW; ++q) {
+            if (!(rlive[p] && clive[q])) continue;
+            product(x[p], y[q], p, q);
+          }
+      }
+    }
+  }
+}
+
+// ---- the same products for few workgroups
+// A grid of at most one workgroup per CU has one wave on a SIMD: nothing covers the latency
+// of a panel's loads, its two barriers and its LDS round trip, and the 16-wide panels above
+// leave the matrix pipe idle two thirds of the time (n = 512, batch 1: 314 us a stage of 92 us
+// of MFMA).  Here a panel is 64 wide (1536 cycles of MFMA a wave) and LDS holds two: while one feeds
+// the products, every k-step stores one element of the next into the other buffer and issues
+// one load of the panel after that, so a panel costs one barrier.  `count` products of the
+// same kind (matrices sa / sb elements apart) run as one sequence of panels, so only the first
+// waits for its loads.  The order of the products of an output is gemm_term's: the same bits.
+constexpr int DW = 64;          // panel width
+constexpr int DWP = DW + 1;
+
+template <int MODE, typename R>
+constexpr int deep_smem() { return 2 * (32 * DWP + (DW * 33 > 32 * DWP ? DW * 33 : 32 * DWP)) * (int)sizeof(typename CT<R>::C); }
+
+// One operand's panels: 32 rows x DW columns (ROWS) or DW rows x 32 columns, 8 elements a thread
+template <bool ROWS, typename C>
+struct DeepPanel {
+  static constexpr int NR = 32 * DW / 256;
+  const char* base;
+  unsigned off[NR];
+  C reg[NR];
+  __device__ __forceinline__ static int k_of(int q, int tid) {
+    const int e = tid + q * 256;
+    return ROWS ? e % DW : e / 32;
+  }
+  __device__ __forceinline__ void start(const C* M, int n, int first, int k0) {
+    base = reinterpret_cast<const char*>(ROWS ? M + (size_t)first * n + k0 : M + (size_t)k0 * n + first);
+  }
+  // element offsets of a panel with `left` values of k in the operator (rows and columns beyond
+  // it read the last valid one)
+  __device__ __forceinline__ void offsets(int n, int first, int left, int tid) {
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+      const int e = tid + q * 256, k = min(k_of(q, tid), left - 1);
+      const int x = min(ROWS ? e / DW : e % 32, n - 1 - first);
+      off[q] = (unsigned)(ROWS ? x * n + k : k * n + x) * (unsigned)sizeof(C);
+    }
+  }
+  __device__ __forceinline__ void load(int q) { reg[q] = *reinterpret_cast<const C*>(base + off[q]); }
+  __device__ __forceinline__ void zero(int left, int tid) {
+#pragma unroll
+    for (int q = 0; q < NR; ++q)
+      if (k_of(q, tid) >= left) {
+        reg[q].x = 0;
+        reg[q].y = 0;
+      }
+  }
+  __device__ __forceinline__ void store(C* sM, int q, int tid) const {
+    const int e = tid + q * 256;
+    sM[ROWS ? (e / DW) * DWP + e % DW : (e / 32) * 33 + e % 32] = reg[q];
+  }
+};
+
+template <int MODE, typename R>
+__device__ __forceinline__ void gemm_deep(const typename CT<R>::C* __restrict__ A, const typename CT<R>::C* __restrict__ B,
+                                          int count, size_t sa, size_t sb, int n, int row0, int col0,
+                                          unsigned char* smem, typename CT<R>::V4& cr, typename CT<R>::V4& ci,
+                                          typename CT<R>::V4& dr, int tid, int wr, int wc, int lr, int lg) {
+  using C = typename CT<R>::C;
+  constexpr int NR = DeepPanel<true, C>::NR;
+  constexpr int ABUF = 32 * DWP, BBUF = DW * 33 > 32 * DWP ? DW * 33 : 32 * DWP;
+  C* sA = reinterpret_cast<C*>(smem);
+  C* sB = sA + 2 * ABUF;
+  const int per = (n + DW - 1) / DW, total = per * count;   // panels
+  DeepPanel<true, C> pa;
+  DeepPanel<MODE != PLAIN, C> pb;
+  // load panel p (past the last one: the last one again, into a buffer nobody reads); the element
+  // offsets change only between whole panels and a product's last, narrower one
+  int width = 0, held = 0;                    // panel width the offsets are for; of the panel in the registers
+  const auto point = [&](int p) {
+    const int x = min(p, total - 1), m = x / per, k0 = (x - m * per) * DW;
+    pa.start(A + m * sa, n, row0, k0);
+    pb.start(B + m * sb, n, col0, k0);
+    const int left = min(DW, n - k0);
+    if (left != width) {
+      pa.offsets(n, row0, left, tid);
+      pb.offsets(n, col0, left, tid);
+      width = left;
+    }
+  };
+  const auto pad = [&]() {                    // zeros beyond a narrower panel's last k
+    if (held < DW) {
+      pa.zero(held, tid);
+      pb.zero(held, tid);
+    }
+    held = width;
+  };
+  __syncthreads();                            // the buffers' previous users are done
+  point(0);
+  held = width;
+#pragma unroll
+  for (int q = 0; q < NR; ++q) {
+    pa.load(q);
+    pb.load(q);
+  }
+  pad();
+#pragma unroll
+  for (int q = 0; q < NR; ++q) {
+    pa.store(sA, q, tid);
+    pb.store(sB, q, tid);
+  }
+  point(1);
+  held = width;
+#pragma unroll
+  for (int q = 0; q < NR; ++q) {
+    pa.load(q);
+    pb.load(q);
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int p = 0; p < total; ++p) {
+    const C* a = sA + (p & 1) * ABUF + (wr * 16 + lr) * DWP + lg;
+    const C* b = sB + (p & 1) * BBUF + (MODE == PLAIN ? lg * 33 + wc * 16 + lr : (wc * 16 + lr) * DWP + lg);
+    C* na = sA + ((p + 1) & 1) * ABUF;
+    C* nb = sB + ((p + 1) & 1) * BBUF;
+    point(p + 2);
+    pad();
+    // one block of k-steps, stores and loads, in this order (the scheduler would move each read down
+    // to its products, whose latency nothing else covers here, and the loads to the end); k-steps
+    // of a narrower panel beyond n multiply zeros
+    constexpr int KS = DW / 4, AHEAD = 3;     // fragments are read three k-steps ahead
+    C x[KS], h[KS];
+#pragma unroll
+    for (int kk = 0; kk < AHEAD; ++kk) {
+      x[kk] = a[4 * kk];
+      h[kk] = b[MODE == PLAIN ? 4 * kk * 33 : 4 * kk];
+    }
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) {
+      if (kk + AHEAD < KS) {
+        x[kk + AHEAD] = a[4 * (kk + AHEAD)];
+        h[kk + AHEAD] = b[MODE == PLAIN ? 4 * (kk + AHEAD) * 33 : 4 * (kk + AHEAD)];
+      }
+      const R as = x[kk].x + x[kk].y;
+      if (MODE == PLAIN) {
+        cr = CT<R>::mfma(x[kk].x, h[kk].x, cr);
+        dr = CT<R>::mfma(x[kk].y, h[kk].y, dr);
+        ci = CT<R>::mfma(as, h[kk].x + h[kk].y, ci);
+      } else if (MODE == NEG_AH) {
+        cr = CT<R>::mfma(-x[kk].x, h[kk].x, cr);
+        dr = CT<R>::mfma(x[kk].y, h[kk].y, dr);
+        ci = CT<R>::mfma(as, h[kk].y - h[kk].x, ci);
+      } else {
+        cr = CT<R>::mfma(x[kk].x, h[kk].y, cr);
+        dr = CT<R>::mfma(x[kk].y, h[kk].x, dr);
+        ci = CT<R>::mfma(as, h[kk].x + h[kk].y, ci);
+      }
+      if (kk < NR) {
+        pa.store(na, kk, tid);
+        pa.load(kk);
+      } else if (kk < 2 * NR) {
+        pb.store(nb, kk - NR, tid);
+        pb.load(kk - NR);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
   }
 }
 
@@ -511,7 +730,7 @@ template <int TILE, int P>
 constexpr bool tk_split() { return P == 1 && TILE == 32; }
 
 // (3xBF16: APS / BPS mark pre-split operands, with row pitch ldp.)
-template <int TILE, int MODE, typename R, int P, bool APS = false, bool BPS = false, bool RAG = false>
+template <int TILE, int MODE, typename R, int P, bool APS = false, bool BPS = false>
 __device__ __forceinline__ void term(const void* __restrict__ A, const void* __restrict__ B, int n, int ldp, int row0,
                                      int col0, unsigned char* smem,
                                      typename CT<R>::V4 (&cr)[TILE / 32][TILE / 32],
@@ -523,11 +742,8 @@ __device__ __forceinline__ void term(const void* __restrict__ A, const void* __r
   } else {
     using C = typename CT<R>::C;
     C* sA = reinterpret_cast<C*>(smem);
-    // interior panels without bounds tests for the per-stage 64-tiles (dense512 FP32: +3.5 %);
-    // the 32-tiles (n = 129 gradient forward: 3.6 % slower) and the persistent ragged kernel
-    // (9.5 % slower) keep the bounds-tested loads
-    gemm_term<TILE, MODE, R, !RAG && TILE == 64>(static_cast<const C*>(A), static_cast<const C*>(B), n, row0, col0, sA,
-                             sA + TILE * KWP, cr, ci, dr, tid, wr, wc, lr, lg, kb, ke);
+    gemm_term<TILE, MODE, R>(static_cast<const C*>(A), static_cast<const C*>(B), n, row0, col0, sA, sA + TILE * KWP, cr,
+                             ci, dr, tid, wr, wc, lr, lg, kb, ke);
   }
 }
 
@@ -580,7 +796,7 @@ __device__ __forceinline__ Geo geometry(int n, int tile_index, int tid) {
 
 // C = H S - S H^dag + i sum_k T_k R_k^dag for operator b (set = b / group), the reductions
 // over k in [kb, ke) (a K-split part; all of them: kb = 0, ke = n).
-template <int TILE, typename R, int P, bool RAG = false>
+template <int TILE, typename R, int P>
 __device__ __forceinline__ void generator_gemms(const TiledArgs& a, int b, const Geo& g, unsigned char* smem,
                                                 typename CT<R>::V4 (&cr)[TILE / 32][TILE / 32],
                                                 typename CT<R>::V4 (&ci)[TILE / 32][TILE / 32], int kb, int ke) {
@@ -600,11 +816,11 @@ __device__ __forceinline__ void generator_gemms(const TiledArgs& a, int b, const
   constexpr bool PS = P == 1;
   const size_t np = (size_t)4 * n * a.ldp;   // u16 elements of one pre-split matrix
   const void* Hop = PS ? static_cast<const void*>(a.hsp + (size_t)set * np) : static_cast<const void*>(H);
-  term<TILE, PLAIN, R, P, PS, false, RAG>(Hop, S, n, a.ldp, g.row0, g.col0, smem, cr, ci, dr, g.tid, g.wr, g.wc, g.lr,
+  term<TILE, PLAIN, R, P, PS, false>(Hop, S, n, a.ldp, g.row0, g.col0, smem, cr, ci, dr, g.tid, g.wr, g.wc, g.lr,
                                           g.lg, kb, ke);
   // one-sided generators (dX/dt = G X, H_eff = i G) have no X H_eff^dag product
   if (!(a.flags & kFlagOneSided))
-    term<TILE, NEG_AH, R, P, false, PS, RAG>(S, Hop, n, a.ldp, g.row0, g.col0, smem, cr, ci, dr, g.tid, g.wr, g.wc,
+    term<TILE, NEG_AH, R, P, false, PS>(S, Hop, n, a.ldp, g.row0, g.col0, smem, cr, ci, dr, g.tid, g.wr, g.wc,
                                              g.lr, g.lg, kb, ke);
   for (int k = 0; k < a.n_dense; ++k) {
     constexpr bool TS = tk_split<TILE, P>();
@@ -614,7 +830,7 @@ __device__ __forceinline__ void generator_gemms(const TiledArgs& a, int b, const
     const size_t rk = (size_t)set * a.n_dense + k;
     const void* Rk = PS ? static_cast<const void*>((a.rsp ? a.rsp : a.lsp) + rk * np)
                         : static_cast<const void*>(static_cast<const C*>(a.rops ? a.rops : a.lops) + rk * nn);
-    term<TILE, I_AH, R, P, TS, PS, RAG>(T, Rk, n, a.ldp, g.row0, g.col0, smem, cr, ci, dr, g.tid, g.wr, g.wc, g.lr,
+    term<TILE, I_AH, R, P, TS, PS>(T, Rk, n, a.ldp, g.row0, g.col0, smem, cr, ci, dr, g.tid, g.wr, g.wc, g.lr,
                                         g.lg, kb, ke);
   }
   finish_terms<TILE, R, P>(cr, ci, dr);
@@ -623,7 +839,7 @@ __device__ __forceinline__ void generator_gemms(const TiledArgs& a, int b, const
 }  // namespace
 
 // One TILE x TILE tile of T[b][k] = L[set][k] @ S[b] (set = b / group).
-template <int TILE, typename R, int P, bool RAG = false>
+template <int TILE, typename R, int P>
 __device__ __forceinline__ void left_tile(const TiledArgs& a, int b, int k, const Geo& g, unsigned char* smem) {
   using C = typename CT<R>::C;
   using V4 = typename CT<R>::V4;
@@ -640,7 +856,7 @@ __device__ __forceinline__ void left_tile(const TiledArgs& a, int b, int k, cons
   const size_t lk = (size_t)set * a.n_dense + k;
   const void* Lk = PS ? static_cast<const void*>(a.lsp + lk * 4 * a.n * a.ldp)
                       : static_cast<const void*>(static_cast<const C*>(a.lops) + lk * nn);
-  term<TILE, PLAIN, R, P, PS, false, RAG>(Lk, static_cast<const C*>(a.s_cur) + (size_t)b * nn, a.n, a.ldp, g.row0,
+  term<TILE, PLAIN, R, P, PS, false>(Lk, static_cast<const C*>(a.s_cur) + (size_t)b * nn, a.n, a.ldp, g.row0,
                                      g.col0, smem, cr, ci, dr, g.tid, g.wr, g.wc, g.lr, g.lg, 0, a.n);
   finish_terms<TILE, R, P>(cr, ci, dr);
   if constexpr (tk_split<TILE, P>()) {
@@ -948,6 +1164,41 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMinWa
   stage_tile_epilogue<TILE, R, P>(a, b, set, idx, g, cr, ci, sRed);
 }
 
+// The stage for few workgroups: 32 x 32 tiles on the deep panels.
+template <typename R>
+__global__ void __launch_bounds__(256) lindblad_stage_deep(TiledArgs a) {
+  using C = typename CT<R>::C;
+  using V4 = typename CT<R>::V4;
+  __shared__ __align__(16) unsigned char smem[deep_smem<PLAIN, R>()];
+  __shared__ double2 sRed[4];
+  const int n = a.n, nc = a.nc;
+  const int tiles = tiles_per_dim(nc, 32) * tiles_per_dim(nc, 32);
+  const int per = tiles + a.border_wgs;
+  const int blk = xcd_block();
+  const int b = blk / per, idx = blk % per;
+  const int set = b / a.group;
+  if (idx >= tiles) {                         // border workgroup (uniform branch)
+    stage_border<R>(a, b, set, idx, tiles, sRed);
+    return;
+  }
+  const size_t nn = (size_t)n * n;
+  const Geo g = geometry<32>(nc, idx, threadIdx.x);
+  const C* H = static_cast<const C*>(a.heff) + (size_t)set * nn;
+  const C* S = static_cast<const C*>(a.s_cur) + (size_t)b * nn;
+  V4 cr[1][1], ci[1][1], dr = V4{0, 0, 0, 0};
+  cr[0][0] = ci[0][0] = dr;
+  gemm_deep<PLAIN, R>(H, S, 1, 0, 0, n, g.row0, g.col0, smem, cr[0][0], ci[0][0], dr, g.tid, g.wr, g.wc, g.lr, g.lg);
+  if (!(a.flags & kFlagOneSided))
+    gemm_deep<NEG_AH, R>(S, H, 1, 0, 0, n, g.row0, g.col0, smem, cr[0][0], ci[0][0], dr, g.tid, g.wr, g.wc, g.lr, g.lg);
+  if (a.n_dense > 0)
+    gemm_deep<I_AH, R>(static_cast<const C*>(a.tbuf) + (size_t)b * a.n_dense * nn,
+                       static_cast<const C*>(a.rops ? a.rops : a.lops) + (size_t)set * a.n_dense * nn, a.n_dense, nn, nn,
+                       n, g.row0, g.col0, smem, cr[0][0], ci[0][0], dr, g.tid, g.wr, g.wc, g.lr, g.lg);
+  ci[0][0] -= cr[0][0] + dr;
+  cr[0][0] -= dr;
+  stage_tile_epilogue<32, R, 0>(a, b, set, idx, g, cr, ci, sRed);
+}
+
 // K-split stage products (a.ks > 1): ks consecutive workgroups per core tile, part p
 // reducing k in [p klen, (p + 1) klen) into its partial sums; lindblad_stage_sum then
 // finishes the stage (and forms the border of the bordered layout).  More workgroups for
@@ -971,7 +1222,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMinWa
 #pragma unroll
     for (int q = 0; q < BW; ++q) cr[p][q] = ci[p][q] = V4{0, 0, 0, 0};
   const int kb = part * a.klen, ke = kb + a.klen < n ? kb + a.klen : n;
-  generator_gemms<TILE, R, P>(a, b, g, smem, cr, ci, kb, ke);
+  // parts beyond n (klen is a multiple of 32) are empty: zeros
+  if (kb < ke) generator_gemms<TILE, R, P>(a, b, g, smem, cr, ci, kb, ke);
   C* Pp = static_cast<C*>(a.part) + ((size_t)part * a.batch + b) * nn;
 #pragma unroll
   for (int p = 0; p < BW; ++p)
@@ -1164,7 +1416,7 @@ lindblad_ragged_persistent(RaggedArgs r) {
           for (int t0 = 0; t0 < tiles; t0 += SG) {
             const int t = t0 + grp;
             const Geo g = geometry<TILE>(n, t < tiles ? t : tiles, ltid);   // tiles: rows >= n
-            left_tile<TILE, float, 0, true>(a, 0, k, g, smem[grp]);
+            left_tile<TILE, float, 0>(a, 0, k, g, smem[grp]);
           }
         }
         if (a.n_dense > 0) __syncthreads();   // T_k complete
@@ -1177,7 +1429,7 @@ lindblad_ragged_persistent(RaggedArgs r) {
           for (int p = 0; p < BW; ++p)
 #pragma unroll
             for (int q = 0; q < BW; ++q) cr[p][q] = ci[p][q] = floatx4{0.f, 0.f, 0.f, 0.f};
-          generator_gemms<TILE, float, 0, true>(a, 0, g, smem[grp], cr, ci, 0, n);
+          generator_gemms<TILE, float, 0>(a, 0, g, smem[grp], cr, ci, 0, n);
 #pragma unroll
           for (int p = 0; p < BW; ++p)
 #pragma unroll
@@ -1253,7 +1505,7 @@ __global__ void __launch_bounds__(256) lindblad_ragged_left(RaggedArgs r, const 
   TiledArgs a = instance_args(r, in);
   a.s_cur = r.work + in.work + (st % 2 == 0 ? 0 : (size_t)in.n * in.n);
   const Geo g = geometry<TILE>(in.n, item % tiles, threadIdx.x);
-  left_tile<TILE, float, 0, true>(a, 0, item / tiles, g, smem);
+  left_tile<TILE, float, 0>(a, 0, item / tiles, g, smem);
 }
 
 // One RK4 stage: list items are the tiles
@@ -1277,7 +1529,7 @@ __global__ void __launch_bounds__(256) lindblad_ragged_stage(RaggedArgs r, const
   for (int p = 0; p < BW; ++p)
 #pragma unroll
     for (int q = 0; q < BW; ++q) cr[p][q] = ci[p][q] = floatx4{0.f, 0.f, 0.f, 0.f};
-  generator_gemms<TILE, float, 0, true>(a, 0, g, smem, cr, ci, 0, n);
+  generator_gemms<TILE, float, 0>(a, 0, g, smem, cr, ci, 0, n);
 #pragma unroll
   for (int p = 0; p < BW; ++p)
 #pragma unroll
@@ -1505,6 +1757,14 @@ hipError_t tiled_apply(TiledArgs a, hipStream_t stream, int tile, bool fp64) {
   return tile == 64 ? apply_impl<64, float>(a, stream) : apply_impl<32, float>(a, stream);
 }
 
+// The stage on the deep panels: one tile per CU at most, and a reduction of whole 64-wide panels or
+// nearly (us per RK4 step, 32-tiles / deep: n = 512 with 16 jump operators 1516 / 1211, FP64 2332 /
+// 2002, without 139 / 123; four n = 256 with 4 274 / 245; n = 500 with 3 424 / 369; but n = 257
+// 81 / 91, n = 400 112 / 114, n = 200 with 2 148 / 165, and at two tiles per CU n = 512 x 2 1950 / 2014).
+static bool deep_stage(int n, long long tiles) {
+  return n >= 256 && tiles <= 256 && cdiv(n, DW) * DW * 25 <= n * 27;
+}
+
 template <int TILE, typename R, int P>
 static hipError_t run_step(TiledArgs a, hipStream_t stream, void* s0, void* s1) {
   const int per = layout(a, TILE);
@@ -1524,6 +1784,12 @@ static hipError_t run_step(TiledArgs a, hipStream_t stream, void* s0, void* s1) 
         hipLaunchKernelGGL((lindblad_stage_part<TILE, R, P>), dim3((per - a.border_wgs) * a.batch * a.ks), dim3(256),
                            0, stream, a);
         hipLaunchKernelGGL((lindblad_stage_sum<TILE, R, P>), dim3(per * a.batch), dim3(256), 0, stream, a);
+        split = true;
+      }
+    }
+    if constexpr (TILE == 32 && P == 0) {
+      if (!split && deep_stage(a.n, (per - a.border_wgs) * a.batch)) {
+        hipLaunchKernelGGL((lindblad_stage_deep<R>), dim3(per * a.batch), dim3(256), 0, stream, a);
         split = true;
       }
     }
@@ -1663,9 +1929,21 @@ size_t tiled_workspace_bytes(int batch, int n, int group, int n_dense, int flags
   return work_layout(batch, n, group, n_dense, flags, fp64, n_eops, rops, tile, ks).total;
 }
 
-int tiled_pick(int batch, int n) {
-  const int t64 = (n + 63) / 64;
-  return ((size_t)batch * t64 * t64 >= 512) ? 64 : 32;
+// 64 x 64 tiles do a quarter of the panel traffic per product but waste more at the edges and hold
+// two waves a SIMD (FP32; FP64 one): they pay from 512 workgroups on, without more padding than
+// 32-tiles, where a stage is mostly dense products.  us per RK4 step, 32 / 64: FP32 16 x n = 512 with
+// 16 jump operators 15900 / 13600, 128 x n = 128 with 4 678 / 642, but 64 x n = 256 without 518 / 528,
+// 256 x n = 100 244 / 297, 128 x n = 129 221 / 286, 64 x n = 200 with 4 1397 / 1849.  The BF16 split
+// products, whose panels are staged at more cost, gain earlier: 64 x n = 192 without 199 / 186, 8 x
+// n = 512 344 / 275, 64 x n = 200 with 4 1248 / 1165, but 128 x n = 129 213 / 238, 64 x n = 160
+// 137 / 171.  Both edges give the same bits, except at n = 32 m + 1, odd m, without dense operators:
+// there the 32-tiles alone use the bordered layout, and the choice stays by the workgroups.
+int tiled_pick(int batch, int n, int n_dense, bool split) {
+  const long long t64 = cdiv(n, 64), e64 = t64 * 64, e32 = 32ll * cdiv(n, 32);
+  if (batch * t64 * t64 < 512) return 32;
+  if (n_dense == 0 && n % 64 == 33) return 64;
+  if (split) return (long long)(2 + n_dense) * n >= 384 && 100 * e64 * e64 <= 135 * e32 * e32 ? 64 : 32;
+  return n_dense >= 3 && e64 == e32 ? 64 : 32;
 }
 
 // Pre-split planes of count n x n complex64 matrices: thread t forms one 16-byte chunk (8

@@ -63,7 +63,7 @@ size_t tiled_workspace_bytes(int batch, int n, int group, int n_dense, int flags
 
 // lime_lindblad_batch.flags bit of one-sided generators (LIME_F_ONE_SIDED)
 constexpr int kFlagOneSided = 0x200;
-int tiled_pick(int batch, int n);
+int tiled_pick(int batch, int n, int n_dense, bool split);
 hipError_t tiled_run(TiledArgs a, int nsteps, int step_offset, int nout, void* work, hipStream_t stream,
                      int tile, TiledPrec prec);
 hipError_t tiled_apply(TiledArgs a, hipStream_t stream, int tile, bool fp64);
