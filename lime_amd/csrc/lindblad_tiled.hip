@@ -605,6 +605,83 @@ struct RowPanel<ROWS, true> {
   }
 };
 
+// A whole panel of ROWS rows x COLS columns in registers, at wave-uniform addresses plus 32-bit offsets
+// (rows or columns beyond the operator read its last one): pairs of complex64 elements, or 16-byte
+// chunks of pre-split planes.
+typedef float float4u __attribute__((ext_vector_type(4), aligned(8)));
+template <int ROWS, bool PRE, int COLS = KB>
+struct FastRows {
+  static constexpr int NP = PanelPairs<ROWS, COLS>::NP;
+  const char* base;
+  size_t step;
+  unsigned off[NP];
+  float4u r[NP];
+  // rows x .., k along the columns
+  __device__ __forceinline__ void init(const void* M, int n, int, int first, int k0, int tid) {
+    base = reinterpret_cast<const char*>(static_cast<const float2*>(M) + (size_t)first * n + k0);
+    step = COLS * sizeof(float2);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int q = tid + 256 * i, x = min(q / (COLS / 2), n - 1 - first);
+      off[i] = (unsigned)(x * n + 2 * (q % (COLS / 2))) * (unsigned)sizeof(float2);
+    }
+  }
+  // k along the rows, columns first .. (n even, so no pair straddles the last column)
+  __device__ __forceinline__ void init_cols(const void* M, int n, int k0, int first, int tid) {
+    base = reinterpret_cast<const char*>(static_cast<const float2*>(M) + (size_t)k0 * n + first);
+    step = (size_t)ROWS * n * sizeof(float2);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int q = tid + 256 * i, x = min(2 * (q % (COLS / 2)), n - 2 - first);
+      off[i] = (unsigned)(q / (COLS / 2) * n + x) * (unsigned)sizeof(float2);
+    }
+  }
+  __device__ __forceinline__ void load() {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) r[i] = *reinterpret_cast<const float4u*>(base + off[i]);
+    base += step;
+  }
+  template <int PITCH, bool NEG>
+  __device__ __forceinline__ void store(u16* sM, int tid) const {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int q = tid + 256 * i;
+      put_pair<ROWS * PITCH, NEG>(sM, q / (COLS / 2) * PITCH + 2 * (q % (COLS / 2)), float2v{r[i].x, r[i].y},
+                                  float2v{r[i].z, r[i].w});
+    }
+  }
+};
+template <int ROWS>
+struct FastRows<ROWS, true, KB> {
+  static constexpr int NC = PanelChunks<ROWS>::NC;
+  const char* base;
+  size_t plane;                               // bytes of one plane
+  unsigned off[NC];
+  u16x8 r[NC];
+  __device__ __forceinline__ void init(const void* M, int n, int ldp, int first, int k0, int tid) {
+    base = reinterpret_cast<const char*>(static_cast<const u16*>(M) + (size_t)first * ldp + k0);
+    plane = (size_t)n * ldp * sizeof(u16);
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int e = (tid + 256 * i) % PanelChunks<ROWS>::PER_PLANE, x = min(e / (KB / 8), n - 1 - first);
+      off[i] = (unsigned)(x * ldp + 8 * (e % (KB / 8))) * (unsigned)sizeof(u16);
+    }
+  }
+  __device__ __forceinline__ void load() {
+    // chunk 256 i + tid lies in plane (256 i + tid) / PER_PLANE, which is wave-uniform
+    static_assert(PanelChunks<ROWS>::PER_PLANE % 64 == 0, "a wave's chunks lie in one plane");
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x & 255) & ~63;
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      r[i] = *reinterpret_cast<const u16x8*>(base + (size_t)((wave + 256 * i) / PanelChunks<ROWS>::PER_PLANE) * plane + off[i]);
+    base += KB * sizeof(u16);
+  }
+  template <int PITCH, bool NEG>
+  __device__ __forceinline__ void store(u16* sM, int tid) const {
+    store_chunks<ROWS, NEG>(sM, r, tid);
+  }
+};
+
 // APS / BPS: the A operand / the B operand of a conjugate-transpose mode comes pre-split
 // (planes with row pitch ldp); otherwise complex64, split while staged.
 template <int TILE, int MODE, bool APS, bool BPS>
@@ -624,6 +701,9 @@ __device__ __forceinline__ void gemm_term_bf3(const void* __restrict__ A, const 
     rlive[p] = row0 + wr * (TILE / 2) + p * 16 < n;
     clive[p] = col0 + wc * (TILE / 2) + p * 16 < n;
   }
+  bool all_live = true;
+#pragma unroll
+  for (int p = 0; p < BW; ++p) all_live = all_live && rlive[p] && clive[p];
   u16* sA = reinterpret_cast<u16*>(smem);
   u16* sB = sA + 4 * APLANE;
   constexpr int BPLANE = MODE == PLAIN ? KB * PB : TILE * PP;
@@ -639,8 +719,97 @@ __device__ __forceinline__ void gemm_term_bf3(const void* __restrict__ A, const 
     if constexpr (MODE == PLAIN) load_pairs<KB, TILE>(static_cast<const float2*>(Bsrc), n, k, col0, rp, tid);
     else rb.load(Bsrc, n, ldp, col0, k, tid);
   };
-  if constexpr (PF) load_panel(kb);
-  for (int k0 = kb; k0 < ke; k0 += KB) {
+  // the fragments of a panel, read from LDS
+  u16x8 a0h[BW], a0l[BW], a1h[BW], a1l[BW], b0h[BW], b0l[BW], b1h[BW], b1l[BW];
+  const auto read_a = [&]() {
+#pragma unroll
+    for (int p = 0; p < BW; ++p) {
+      const int o = (wr * (TILE / 2) + p * 16 + lr) * PP + 8 * lg;
+      a0h[p] = *reinterpret_cast<const u16x8*>(sA + o);
+      a0l[p] = *reinterpret_cast<const u16x8*>(sA + APLANE + o);
+      a1h[p] = *reinterpret_cast<const u16x8*>(sA + 2 * APLANE + o);
+      a1l[p] = *reinterpret_cast<const u16x8*>(sA + 3 * APLANE + o);
+    }
+  };
+  const auto read_b = [&](int q) {
+    if constexpr (MODE == PLAIN) {
+      // transposed reads: lane (lg, lr) loads plane row 8 lg + lr / 4 (+ 4), columns
+      // c + 4 (lr % 4) .. + 3 of the block's 16 columns
+      const int o = (8 * lg + (lr >> 2)) * PB + wc * (TILE / 2) + q * 16 + 4 * (lr & 3);
+      u16x8 f[4];
+#pragma unroll
+      for (int pl = 0; pl < 4; ++pl) {
+        const u16* base = sB + pl * BPLANE + o;
+        const short4v x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(base));
+        const short4v y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(base + 4 * PB));
+        f[pl] = u16x8{(u16)x[0], (u16)x[1], (u16)x[2], (u16)x[3], (u16)y[0], (u16)y[1], (u16)y[2], (u16)y[3]};
+      }
+      b0h[q] = f[0];
+      b0l[q] = f[1];
+      b1h[q] = f[2];
+      b1l[q] = f[3];
+    } else {
+      const int o = (wc * (TILE / 2) + q * 16 + lr) * PP + 8 * lg;
+      b0h[q] = *reinterpret_cast<const u16x8*>(sB + o);
+      b0l[q] = *reinterpret_cast<const u16x8*>(sB + BPLANE + o);
+      b1h[q] = *reinterpret_cast<const u16x8*>(sB + 2 * BPLANE + o);
+      b1l[q] = *reinterpret_cast<const u16x8*>(sB + 3 * BPLANE + o);
+    }
+  };
+  int k0 = kb;
+  // whole panels of blocks inside the operator: loads at one wave-uniform address plus 32-bit offsets
+  // formed once (as Panel above), and one basic block of products, the accumulators in turn so that no
+  // MFMA waits for the one before it (each accumulator's own order is that of the tested loop).  us per
+  // RK4 step, tested / here: 16 x n = 512 with 16 jump operators 7980 / 7300, one of them (32-tiles) 1000
+  // / 945, 4 x n = 500 with 4 (64) 1100 / 823, 16 x n = 256 with 4 (64) 465 / 419, 64 x n = 192 (64) 188 / 184.
+  if (all_live && (MODE != PLAIN || n % 2 == 0)) {
+    FastRows<TILE, APS> fa;
+    FastRows<MODE == PLAIN ? KB : TILE, BPS, MODE == PLAIN ? TILE : KB> fb;
+    fa.init(A, n, ldp, row0, kb, tid);
+    if constexpr (MODE == PLAIN) fb.init_cols(Bsrc, n, kb, col0, tid);
+    else fb.init(Bsrc, n, ldp, col0, kb, tid);
+    const auto load_fast = [&]() {
+      fa.load();
+      fb.load();
+    };
+    if (PF && k0 < ke && k0 + KB <= n) load_fast();
+    for (; k0 < ke && k0 + KB <= n; k0 += KB) {
+      if constexpr (!PF) load_fast();
+      __syncthreads();
+      fa.template store<PP, false>(sA, tid);
+      fb.template store<MODE == PLAIN ? PB : PP, MODE == NEG_AH>(sB, tid);
+      __syncthreads();
+      if constexpr (PF) {
+        if (k0 + KB < ke && k0 + 2 * KB <= n) load_fast();
+      }
+      __builtin_amdgcn_s_setprio(1);
+      read_a();
+#pragma unroll
+      for (int q = 0; q < BW; ++q) {
+        read_b(q);
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+          for (int t = 0; t < 3; ++t)         // lo hi, hi lo, hi hi
+#pragma unroll
+            for (int p = 0; p < BW; ++p) {
+              const u16x8 x0 = t == 0 ? a0l[p] : a0h[p], x1 = t == 0 ? a1l[p] : a1h[p];
+              const u16x8 y0 = t == 1 ? b0l[q] : b0h[q], y1 = t == 1 ? b1l[q] : b1h[q];
+              if (half == 0) {
+                cr[p][q] = mfma_bf(x0, MODE == I_AH ? y1 : y0, cr[p][q]);
+                ci[p][q] = mfma_bf(x0, MODE == I_AH ? y0 : y1, ci[p][q]);
+              } else {
+                dr[p][q] = mfma_bf(x1, MODE == I_AH ? y0 : y1, dr[p][q]);
+                ci[p][q] = mfma_bf(x1, MODE == I_AH ? y1 : y0, ci[p][q]);
+              }
+            }
+      }
+      __builtin_amdgcn_s_setprio(0);
+    }
+  }
+  if (k0 >= ke) return;
+  if constexpr (PF) load_panel(k0);
+  for (; k0 < ke; k0 += KB) {
     if constexpr (!PF) load_panel(k0);
     __syncthreads();                          // previous panel fully consumed
     ra.template store<false>(sA, tid);
@@ -654,41 +823,9 @@ __device__ __forceinline__ void gemm_term_bf3(const void* __restrict__ A, const 
     // over waves staging the next panel (dense512: +2.5 %; the FP32 terms measured 0.3 %
     // slower with it)
     __builtin_amdgcn_s_setprio(1);
-    u16x8 a0h[BW], a0l[BW], a1h[BW], a1l[BW], b0h[BW], b0l[BW], b1h[BW], b1l[BW];
+    read_a();
 #pragma unroll
-    for (int p = 0; p < BW; ++p) {
-      const int o = (wr * (TILE / 2) + p * 16 + lr) * PP + 8 * lg;
-      a0h[p] = *reinterpret_cast<const u16x8*>(sA + o);
-      a0l[p] = *reinterpret_cast<const u16x8*>(sA + APLANE + o);
-      a1h[p] = *reinterpret_cast<const u16x8*>(sA + 2 * APLANE + o);
-      a1l[p] = *reinterpret_cast<const u16x8*>(sA + 3 * APLANE + o);
-    }
-#pragma unroll
-    for (int q = 0; q < BW; ++q) {
-      if constexpr (MODE == PLAIN) {
-        // transposed reads: lane (lg, lr) loads plane row 8 lg + lr / 4 (+ 4), columns
-        // c + 4 (lr % 4) .. + 3 of the block's 16 columns
-        const int o = (8 * lg + (lr >> 2)) * PB + wc * (TILE / 2) + q * 16 + 4 * (lr & 3);
-        u16x8 f[4];
-#pragma unroll
-        for (int pl = 0; pl < 4; ++pl) {
-          const u16* base = sB + pl * BPLANE + o;
-          const short4v x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(base));
-          const short4v y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(base + 4 * PB));
-          f[pl] = u16x8{(u16)x[0], (u16)x[1], (u16)x[2], (u16)x[3], (u16)y[0], (u16)y[1], (u16)y[2], (u16)y[3]};
-        }
-        b0h[q] = f[0];
-        b0l[q] = f[1];
-        b1h[q] = f[2];
-        b1l[q] = f[3];
-      } else {
-        const int o = (wc * (TILE / 2) + q * 16 + lr) * PP + 8 * lg;
-        b0h[q] = *reinterpret_cast<const u16x8*>(sB + o);
-        b0l[q] = *reinterpret_cast<const u16x8*>(sB + BPLANE + o);
-        b1h[q] = *reinterpret_cast<const u16x8*>(sB + 2 * BPLANE + o);
-        b1l[q] = *reinterpret_cast<const u16x8*>(sB + 3 * BPLANE + o);
-      }
-    }
+    for (int q = 0; q < BW; ++q) read_b(q);
 #pragma unroll
     for (int p = 0; p < BW; ++p)
 #pragma unroll
@@ -830,8 +967,12 @@ __device__ __forceinline__ void generator_gemms(const TiledArgs& a, int b, const
     const size_t rk = (size_t)set * a.n_dense + k;
     const void* Rk = PS ? static_cast<const void*>((a.rsp ? a.rsp : a.lsp) + rk * np)
                         : static_cast<const void*>(static_cast<const C*>(a.rops ? a.rops : a.lops) + rk * nn);
-    term<TILE, I_AH, R, P, TS, PS>(T, Rk, n, a.ldp, g.row0, g.col0, smem, cr, ci, dr, g.tid, g.wr, g.wc, g.lr,
-                                        g.lg, kb, ke);
+    // 3xBF16: the thread index is opaque, so the panels' offsets are formed per term instead of being
+    // held (and spilled: 21 registers of the 64-tiles) across the loop
+    int tid = g.tid;
+    if constexpr (P == 1) asm volatile("" : "+v"(tid));
+    term<TILE, I_AH, R, P, TS, PS>(T, Rk, n, a.ldp, g.row0, g.col0, smem, cr, ci, dr, tid, g.wr, g.wc, g.lr, g.lg, kb,
+                                   ke);
   }
   finish_terms<TILE, R, P>(cr, ci, dr);
 }
@@ -860,8 +1001,8 @@ __device__ __forceinline__ void left_tile(const TiledArgs& a, int b, int k, cons
                                      g.col0, smem, cr, ci, dr, g.tid, g.wr, g.wc, g.lr, g.lg, 0, a.n);
   finish_terms<TILE, R, P>(cr, ci, dr);
   if constexpr (tk_split<TILE, P>()) {
-    // 3xBF16, 32-tiles: T_k goes out as split planes (row pitch ldp; the columns n .. ldp - 1
-    // hold the products with the zero columns beyond n, i.e. zeros)
+    // 3xBF16, 32-tiles: T_k goes out as split planes (row pitch ldp, zeros in the columns n ..
+    // ldp - 1)
     const size_t plane = (size_t)a.n * a.ldp;
     u16* T = static_cast<u16*>(a.tbuf) + ((size_t)b * a.n_dense + k) * 4 * plane;
 #pragma unroll
@@ -874,7 +1015,7 @@ __device__ __forceinline__ void left_tile(const TiledArgs& a, int b, int k, cons
           const int j = g.col0 + g.wc * (TILE / 2) + q * 16 + g.lr;
           if (i < a.n && j < a.ldp) {
             unsigned h, l;
-            split2(cr[p][q][v], ci[p][q][v], h, l);
+            split2(j < a.n ? cr[p][q][v] : 0.f, j < a.n ? ci[p][q][v] : 0.f, h, l);
             u16* t = T + (size_t)i * a.ldp + j;
             t[0] = (u16)h;
             t[plane] = (u16)l;
