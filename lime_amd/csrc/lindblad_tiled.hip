@@ -760,8 +760,8 @@ __device__ __forceinline__ void gemm_term_bf3(const void* __restrict__ A, const 
   // whole panels of blocks inside the operator: loads at one wave-uniform address plus 32-bit offsets
   // formed once (as Panel above), and one basic block of products, the accumulators in turn so that no
   // MFMA waits for the one before it (each accumulator's own order is that of the tested loop).  us per
-  // RK4 step, tested / here: 16 x n = 512 with 16 jump operators 7980 / 7300, one of them (32-tiles) 1000
-  // / 945, 4 x n = 500 with 4 (64) 1100 / 823, 16 x n = 256 with 4 (64) 465 / 419, 64 x n = 192 (64) 188 / 184.
+  // RK4 step, tested / here: 16 x n = 512 with 16 jump operators 7980 / 7300, one of them (32-tiles) 1010
+  // / 970, 4 x n = 500 with 4 (64) 1100 / 823, 16 x n = 256 with 4 (64) 465 / 419, 64 x n = 192 (64) 188 / 184.
   if (all_live && (MODE != PLAIN || n % 2 == 0)) {
     FastRows<TILE, APS> fa;
     FastRows<MODE == PLAIN ? KB : TILE, BPS, MODE == PLAIN ? TILE : KB> fb;
