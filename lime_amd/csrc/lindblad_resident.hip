@@ -1087,6 +1087,7 @@ hipError_t resident_launch(const ResidentArgs& args, int variant, hipStream_t st
   ResidentArgs a = args;
   if (variant < 0 || variant >= resident_variants(a.n, a.n_dense)) return hipErrorInvalidValue;
   if (small_eligible(a)) return small_launch(a, stream);
+  if (variant == 0 && edge_eligible(a)) return edge_launch(a, stream);
   size_t lds = resident_lds_bytes(a.n, variant, a.n_dense, a.n_eops);
   if (a.n_dense > 0) {
     a.op_pitch = dense_pitch(a.n, variant, a.n_dense, a.n_eops, a.rops != nullptr, a.batch);

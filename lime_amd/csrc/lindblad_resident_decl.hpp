@@ -37,6 +37,11 @@ hipError_t resident_launch(const ResidentArgs& a, int variant, hipStream_t strea
 bool small_eligible(const ResidentArgs& a);
 hipError_t small_launch(const ResidentArgs& a, hipStream_t stream);
 
+// Dense jump operators at n = 16 m + 1 .. 4 (lindblad_edge.hip): core on MFMA, the last rows and
+// columns on the vector units; the bits of the resident kernel's default shape.
+bool edge_eligible(const ResidentArgs& a);
+hipError_t edge_launch(const ResidentArgs& a, hipStream_t stream);
+
 // 3xBF16 split-product resident kernel (lindblad_resident_bf3.hip): bordered n = 33, 49, 65
 // without dense operators; one launch shape
 bool resident_bf3_eligible(int n, int n_dense);
