@@ -684,7 +684,7 @@ struct FastRows<ROWS, true, KB> {
 
 // APS / BPS: the A operand / the B operand of a conjugate-transpose mode comes pre-split
 // (planes with row pitch ldp); otherwise complex64, split while staged.
-template <int TILE, int MODE, bool APS, bool BPS>
+template <int TILE, int MODE, bool APS, bool BPS, bool WHOLE>
 __device__ __forceinline__ void gemm_term_bf3(const void* __restrict__ A, const void* __restrict__ Bsrc, int n, int ldp,
                                               int row0, int col0, unsigned char* smem,
                                               floatx4 (&cr)[TILE / 32][TILE / 32],
@@ -757,12 +757,10 @@ __device__ __forceinline__ void gemm_term_bf3(const void* __restrict__ A, const 
     }
   };
   int k0 = kb;
-  // whole panels of blocks inside the operator: loads at one wave-uniform address plus 32-bit offsets
-  // formed once (as Panel above), and one basic block of products, the accumulators in turn so that no
-  // MFMA waits for the one before it (each accumulator's own order is that of the tested loop).  us per
-  // RK4 step, tested / here: 16 x n = 512 with 16 jump operators 7980 / 7300, one of them (32-tiles) 1010
-  // / 970, 4 x n = 500 with 4 (64) 1100 / 823, 16 x n = 256 with 4 (64) 465 / 419, 64 x n = 192 (64) 188 / 184.
-  if (all_live && (MODE != PLAIN || n % 2 == 0)) {
+  // WHOLE: whole panels of blocks inside the operator: loads at one wave-uniform address plus 32-bit
+  // offsets formed once (as Panel above), and one basic block of products, the accumulators in turn so
+  // that no MFMA waits for the one before it (each accumulator's own order is that of the tested loop)
+  if (WHOLE && all_live && (MODE != PLAIN || n % 2 == 0)) {
     FastRows<TILE, APS> fa;
     FastRows<MODE == PLAIN ? KB : TILE, BPS, MODE == PLAIN ? TILE : KB> fb;
     fa.init(A, n, ldp, row0, kb, tid);
@@ -807,7 +805,7 @@ __device__ __forceinline__ void gemm_term_bf3(const void* __restrict__ A, const 
       __builtin_amdgcn_s_setprio(0);
     }
   }
-  if (k0 >= ke) return;
+  if (WHOLE && k0 >= ke) return;
   if constexpr (PF) load_panel(k0);
   for (; k0 < ke; k0 += KB) {
     if constexpr (!PF) load_panel(k0);
@@ -850,12 +848,12 @@ __device__ __forceinline__ void gemm_term_bf3(const void* __restrict__ A, const 
 // Waves per SIMD the compiler must leave room for: the 64 x 64 3xBF16 kernels would take
 // more than 168 VGPRs with the interior-panel load path and drop to 2 waves per SIMD.
 template <int TILE, int P>
-constexpr int kMinWaves = (TILE == 64 && P == 1) ? 3 : 1;
+constexpr int kMinWaves = (TILE == 64 && P != 0) ? 3 : 1;
 
 // LDS bytes of a GEMM-staging area.
 template <int TILE, typename R, int P>
 constexpr int smem_bytes() {
-  return P == 1 ? (4 * TILE * PP + 4 * (KB * pb_pitch<TILE>() > TILE * PP ? KB * pb_pitch<TILE>() : TILE * PP)) * 2
+  return P != 0 ? (4 * TILE * PP + 4 * (KB * pb_pitch<TILE>() > TILE * PP ? KB * pb_pitch<TILE>() : TILE * PP)) * 2
                 : (TILE * KWP + smem_b<TILE>()) * (int)sizeof(typename CT<R>::C);
 }
 
@@ -864,7 +862,7 @@ constexpr int smem_bytes() {
 // (dense512 batch 1: +16 %); the 64-tiles keep complex64 (their 4x more 2-byte plane stores
 // cost 2.6 % at batch 32).
 template <int TILE, int P>
-constexpr bool tk_split() { return P == 1 && TILE == 32; }
+constexpr bool tk_split() { return P != 0 && TILE == 32; }
 
 // (3xBF16: APS / BPS mark pre-split operands, with row pitch ldp.)
 template <int TILE, int MODE, typename R, int P, bool APS = false, bool BPS = false>
@@ -874,8 +872,8 @@ __device__ __forceinline__ void term(const void* __restrict__ A, const void* __r
                                      typename CT<R>::V4 (&ci)[TILE / 32][TILE / 32],
                                      typename CT<R>::V4 (&dr)[TILE / 32][TILE / 32], int tid, int wr, int wc,
                                      int lr, int lg, int kb, int ke) {
-  if constexpr (P == 1) {
-    gemm_term_bf3<TILE, MODE, APS, BPS>(A, B, n, ldp, row0, col0, smem, cr, ci, dr, tid, wr, wc, lr, lg, kb, ke);
+  if constexpr (P != 0) {
+    gemm_term_bf3<TILE, MODE, APS, BPS, P == 2>(A, B, n, ldp, row0, col0, smem, cr, ci, dr, tid, wr, wc, lr, lg, kb, ke);
   } else {
     using C = typename CT<R>::C;
     C* sA = reinterpret_cast<C*>(smem);
@@ -950,7 +948,7 @@ __device__ __forceinline__ void generator_gemms(const TiledArgs& a, int b, const
     for (int q = 0; q < TILE / 32; ++q) dr[p][q] = V4{0, 0, 0, 0};
   // 3xBF16: H_eff, R_k (pre-split once per call) and, for 32-tiles, T_k (written split)
   // from planes
-  constexpr bool PS = P == 1;
+  constexpr bool PS = P != 0;
   const size_t np = (size_t)4 * n * a.ldp;   // u16 elements of one pre-split matrix
   const void* Hop = PS ? static_cast<const void*>(a.hsp + (size_t)set * np) : static_cast<const void*>(H);
   term<TILE, PLAIN, R, P, PS, false>(Hop, S, n, a.ldp, g.row0, g.col0, smem, cr, ci, dr, g.tid, g.wr, g.wc, g.lr,
@@ -970,7 +968,7 @@ __device__ __forceinline__ void generator_gemms(const TiledArgs& a, int b, const
     // 3xBF16: the thread index is opaque, so the panels' offsets are formed per term instead of being
     // held (and spilled: 21 registers of the 64-tiles) across the loop
     int tid = g.tid;
-    if constexpr (P == 1) asm volatile("" : "+v"(tid));
+    if constexpr (P == 2) asm volatile("" : "+v"(tid));
     term<TILE, I_AH, R, P, TS, PS>(T, Rk, n, a.ldp, g.row0, g.col0, smem, cr, ci, dr, tid, g.wr, g.wc, g.lr, g.lg, kb,
                                    ke);
   }
@@ -993,7 +991,7 @@ __device__ __forceinline__ void left_tile(const TiledArgs& a, int b, int k, cons
 #pragma unroll
     for (int q = 0; q < BW; ++q) cr[p][q] = ci[p][q] = dr[p][q] = V4{0, 0, 0, 0};
   // 3xBF16: L_k from its pre-split planes
-  constexpr bool PS = P == 1;
+  constexpr bool PS = P != 0;
   const size_t lk = (size_t)set * a.n_dense + k;
   const void* Lk = PS ? static_cast<const void*>(a.lsp + lk * 4 * a.n * a.ldp)
                       : static_cast<const void*>(static_cast<const C*>(a.lops) + lk * nn);
@@ -1924,7 +1922,7 @@ static hipError_t run_step(TiledArgs a, hipStream_t stream, void* s0, void* s1) 
       if (a.ks > 1) {
         hipLaunchKernelGGL((lindblad_stage_part<TILE, R, P>), dim3((per - a.border_wgs) * a.batch * a.ks), dim3(256),
                            0, stream, a);
-        hipLaunchKernelGGL((lindblad_stage_sum<TILE, R, P>), dim3(per * a.batch), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((lindblad_stage_sum<TILE, R, (P != 0)>), dim3(per * a.batch), dim3(256), 0, stream, a);
         split = true;
       }
     }
@@ -2115,6 +2113,17 @@ __global__ void __launch_bounds__(256) split_planes(const float2* __restrict__ s
   *reinterpret_cast<uint4*>(d + 3 * plane) = make_uint4(yl[0], yl[1], yl[2], yl[3]);
 }
 
+// 3xBF16 with the panels inside the operator loaded without tests (the WHOLE products).  The panel after
+// the last whole one runs the tested loop, whose first load nothing hides, and at odd n the rows of S
+// cannot be read in pairs, so it pays without a remainder, or where the whole panels are many.  us per RK4
+// step, tested / whole: n = 64 x 256 with 4 jump operators 190 / 179, n = 128 x 32 with 4 169 / 161, n = 222
+// x 32 188 / 167, n = 274 x 8 with 4 397 / 382, 512 x 16 with 16 7980 / 7300, but n = 44 x 1024 with 2 367 / 392,
+// n = 66 x 128 with 4 244 / 262, n = 144 x 32 with 2 199 / 206, n = 258 x 16 with 2 400 / 408, odd n = 129 x 16 with
+// 4 175 / 184.
+static bool whole_panels(int n) {
+  return n % KB == 0 || (n % 2 == 0 && (n >= 288 || (n >= 192 && n % KB >= 16)));
+}
+
 template <typename R, int P>
 static hipError_t run_all(TiledArgs a, int nsteps, int step_offset, int nout, void* work, hipStream_t stream,
                           int tile) {
@@ -2126,7 +2135,7 @@ static hipError_t run_all(TiledArgs a, int nsteps, int step_offset, int nout, vo
   a.klen = wl.klen;
   a.part = a.ks > 1 ? static_cast<void*>(static_cast<unsigned char*>(work) + wl.part) : nullptr;
   unsigned char* base = static_cast<unsigned char*>(work);
-  if constexpr (P == 1) {
+  if constexpr (P != 0) {
     // split the constant operators once per call: H_eff, then L_k, then R_k
     unsigned short* sp = reinterpret_cast<unsigned short*>(base + wl.split);
     const size_t np = (size_t)4 * a.n * wl.ldp;
@@ -2232,7 +2241,9 @@ hipError_t tiled_run(TiledArgs a, int nsteps, int step_offset, int nout, void* w
                      int tile, TiledPrec prec) {
   switch (prec) {
     case TiledPrec::FP64: return run_all<double, 0>(a, nsteps, step_offset, nout, work, stream, tile);
-    case TiledPrec::SPLIT_BF16: return run_all<float, 1>(a, nsteps, step_offset, nout, work, stream, tile);
+    case TiledPrec::SPLIT_BF16:
+      return whole_panels(a.n) ? run_all<float, 2>(a, nsteps, step_offset, nout, work, stream, tile)
+                               : run_all<float, 1>(a, nsteps, step_offset, nout, work, stream, tile);
     default: return run_all<float, 0>(a, nsteps, step_offset, nout, work, stream, tile);
   }
 }

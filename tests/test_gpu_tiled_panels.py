@@ -45,6 +45,19 @@ def test_tiles_agree_bit_for_bit_and_with_fp64(n, kd, precision):
         assert float((_run(n, 2, kd, precision, v) - ref).abs().max()) < tol, v
 
 
+@pytest.mark.parametrize("n,kd", [(128, 2), (130, 1), (160, 0), (190, 1), (192, 1), (194, 1), (206, 0), (208, 1), (223, 1),
+                                  (224, 0), (258, 1), (286, 0), (288, 1), (289, 0), (290, 1), (322, 0)])
+def test_split_products_at_the_sizes_where_the_panel_loads_change(n, kd):
+    """3xBF16 with untested loads (no remainder panel, or many whole ones at even n) and with tested ones.
+    The split keeps 16 bits of an element, 7.6e-6; two steps of dt 0.05 whose derivative is of the order of
+    the state and whose n (2 + kd) errors average: under 1e-6 of the largest element."""
+    small = _run(n, 2, kd, "3xbf16", 1)
+    assert torch.equal(small, _run(n, 2, kd, "3xbf16", 2)) or (kd == 0 and n % 64 == 33)
+    ref = _run(n, 2, kd, "fp64", 1)
+    for v in (0, 1, 3, 4):
+        assert float((_run(n, 2, kd, "3xbf16", v) - ref).abs().max()) < 1e-6 * float(ref.abs().max()), v
+
+
 @pytest.mark.parametrize("one_sided", [False, True])
 @pytest.mark.parametrize("precision", ["fp32", "fp64"])
 @pytest.mark.parametrize("n,kd", [(256, 0), (256, 3), (305, 2), (320, 1), (500, 2), (512, 1)])
