@@ -2069,19 +2069,27 @@ size_t tiled_workspace_bytes(int batch, int n, int group, int n_dense, int flags
 }
 
 // 64 x 64 tiles do a quarter of the panel traffic per product but waste more at the edges and hold
-// two waves a SIMD (FP32; FP64 one): they pay from 512 workgroups on, without more padding than
-// 32-tiles, where a stage is mostly dense products.  us per RK4 step, 32 / 64: FP32 16 x n = 512 with
-// 16 jump operators 15900 / 13600, 128 x n = 128 with 4 678 / 642, but 64 x n = 256 without 518 / 528,
-// 256 x n = 100 244 / 297, 128 x n = 129 221 / 286, 64 x n = 200 with 4 1397 / 1849.  The BF16 split
-// products, whose panels are staged at more cost, gain earlier: 64 x n = 192 without 199 / 186, 8 x
-// n = 512 344 / 275, 64 x n = 200 with 4 1248 / 1165, but 128 x n = 129 213 / 238, 64 x n = 160
-// 137 / 171.  Both edges give the same bits, except at n = 32 m + 1, odd m, without dense operators:
-// there the 32-tiles alone use the bordered layout, and the choice stays by the workgroups.
+// fewer waves a SIMD: they pay from 512 workgroups on.  FP32 and FP64 (two waves a SIMD, FP64 one): without
+// more padding than 32-tiles, where a stage is mostly dense products.  us per RK4 step, 32 / 64: 16 x n = 512
+// with 16 jump operators 15900 / 13600, 128 x n = 128 with 4 678 / 642, but 64 x n = 256 without 518 / 528,
+// 256 x n = 100 244 / 297, 128 x n = 129 221 / 286, 64 x n = 200 with 4 1397 / 1849.
+// 3xBF16: a CU holds 3 workgroups of 64-tiles or 4 of 32-tiles, so the time goes in rounds of 768 or
+// 1024, and a round of 64-tiles costs 2.5 of the other, 2 with jump operators where the padding is about
+// the same (the traffic of T_k and R_k), less from n = 256 on.  n = 100 without jump operators: 1440
+// 64-tiles (1.9 rounds) take 0.90 of the 32-tiles' time, n = 124 with 936 (1.2) 1.27, n = 64 with 879 1.34,
+// with 579 and 4 jump operators 0.88; n = 96 (36 for 9 tiles) 1.60 without, 1.24 with 4; 8 x n = 512 0.80.
+// Both edges give the same bits, except at n = 32 m + 1, odd m, without dense operators: there the
+// 32-tiles alone use the bordered layout, and the choice stays by the workgroups.
 int tiled_pick(int batch, int n, int n_dense, bool split) {
-  const long long t64 = cdiv(n, 64), e64 = t64 * 64, e32 = 32ll * cdiv(n, 32);
-  if (batch * t64 * t64 < 512) return 32;
+  const long long n64 = cdiv(n, 64), n32 = cdiv(n, 32), e64 = n64 * 64, e32 = n32 * 32;
+  const long long t64 = batch * n64 * n64, t32 = batch * n32 * n32;
+  if (t64 < 512) return 32;
   if (n_dense == 0 && n % 64 == 33) return 64;
-  if (split) return (long long)(2 + n_dense) * n >= 384 && 100 * e64 * e64 <= 135 * e32 * e32 ? 64 : 32;
+  if (split) {
+    if (n >= 256) return 64;
+    const int half_cost = n_dense == 0 || 100 * e64 * e64 > 145 * e32 * e32 ? 5 : 4;
+    return half_cost * ((t64 + 767) / 768) <= 2 * ((t32 + 1023) / 1024) ? 64 : 32;
+  }
   return n_dense >= 3 && e64 == e32 ? 64 : 32;
 }
 
