@@ -54,7 +54,7 @@ __device__ __forceinline__ void stage_operator(float2* dst, const float2* __rest
 // with row pitches PA and PB.  The reduction runs over k < ke (operands are zero beyond n).
 // sA / sB may be read up to 4 columns / rows past ke (padding, or the spare LDS after each
 // buffer).
-template <int BPW, int MODE>
+template <int BPW, int MODE, int KS>
 __device__ __forceinline__ void lds_gemm(const float2* sA, int PA, const float2* sB, int PB, const int (&trow)[BPW],
                                          const int (&tcol)[BPW], int lr, int lg, int ke, floatx4 (&cr)[BPW],
                                          floatx4 (&ci)[BPW]) {
@@ -70,8 +70,8 @@ __device__ __forceinline__ void lds_gemm(const float2* sA, int PA, const float2*
     x[u] = sA[oA[u]];
     y[u] = sB[oB[u]];
   }
-#pragma unroll 2
-  for (int k0 = 0; k0 < ke; k0 += 4) {
+#pragma unroll (KS > 0 ? KS : 2)
+  for (int k0 = 0; k0 < (KS > 0 ? 4 * KS : ke); k0 += 4) {
     float2 xn[BPW], yn[BPW];
 #pragma unroll
     for (int u = 0; u < BPW; ++u) {
@@ -103,7 +103,7 @@ __device__ __forceinline__ void lds_gemm(const float2* sA, int PA, const float2*
 
 // One loop over both: C += i T R^dag (into cr, ci; T and R^dag as MODE 2 of lds_gemm) and
 // U += L S (into tr, ti; MODE 0), each with lds_gemm's order of products.
-template <int BPW>
+template <int BPW, int KS>
 __device__ __forceinline__ void lds_gemm_pair(const float2* sT, int PT, const float2* sR, const float2* sL, int PO,
                                               const float2* sS, int PS, const int (&trow)[BPW], const int (&tcol)[BPW],
                                               int lr, int lg, int ke, floatx4 (&cr)[BPW], floatx4 (&ci)[BPW],
@@ -121,8 +121,8 @@ __device__ __forceinline__ void lds_gemm_pair(const float2* sT, int PT, const fl
     z[u] = sL[oL[u]];
     h[u] = sS[oS[u]];
   }
-#pragma unroll 2
-  for (int k0 = 0; k0 < ke; k0 += 4) {
+#pragma unroll (KS > 0 ? KS : 2)
+  for (int k0 = 0; k0 < (KS > 0 ? 4 * KS : ke); k0 += 4) {
     float2 xn[BPW], yn[BPW], zn[BPW], hn[BPW];
 #pragma unroll
     for (int u = 0; u < BPW; ++u) {
@@ -166,7 +166,16 @@ __device__ __forceinline__ void lds_gemm_pair(const float2* sT, int PT, const fl
 // operand, and cost a launch, for one step's work.
 // RES (dense jump operators): every L_k and R_k stays in LDS for the launch instead of being
 // staged through one buffer in each stage.
-template <int NB, int W, int BPW, int MINW, bool DENSE, bool REC, bool BRD, bool DB, bool DRV, bool RES>
+//
+// KS > 0: the reduction takes KS k-steps, known when the kernel is built, and its loops are unrolled.
+// With a trip count read at run time the fragment reads of step k0 + 4 are not kept in front of the MFMAs
+// of step k0, and a k-step of 8 MFMAs (256 cycles) took 460 (n = 24, by the cycle counter).  The
+// registers of an unrolled loop still fit, but for NB = 4 with resident operands and for the bordered
+// kernels of n = 65, which spill; unrolled, the other bordered kernels are 1 - 4 % slower.  us per RK4 step,
+// run time / built in, same bits: n = 24 with 8 sandwich terms 48 / 35, n = 32 with 4 jump operators 33 / 25,
+// n = 48 with 4 106 / 90, 2048 of them 975 / 833, n = 64 with 4 191 / 162; without, n = 32 8.1 / 7.2, n = 64
+// 36.0 / 33.5, 4096 of them 588 / 546, 1200 of n = 80 (two tiles a wave, by 2) 434 / 421.
+template <int NB, int W, int BPW, int MINW, bool DENSE, bool REC, bool BRD, bool DB, bool DRV, bool RES, int KS = 0>
 __device__ __forceinline__ void resident_body(const ResidentArgs& a) {
   // LDS rows / columns held: bordered layouts hold the core, the border index and 7 zero
   // ones (the reductions and the fragment prefetch read up to index 16 (NB - 1) + 7)
@@ -233,7 +242,7 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a) {
   const int lr = lane & 15;
   const int lg = lane >> 4;
   // reduction extent: operands are zero beyond n, so round n up to the MFMA k-step
-  const int ke = BRD ? NC + 4 : ((n + 3) & ~3);
+  const int ke = BRD ? NC + 4 : KS > 0 ? 4 * KS : ((n + 3) & ~3);
 
   // ---- stage H_eff into LDS (zero padded to NP); bordered: S is zeroed too, since its
   // padding is not covered by any owner
@@ -455,7 +464,7 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a) {
             }
           }
         }
-#pragma unroll 2
+#pragma unroll (KS > 0 && BPW == 1 ? KS : 2)
         for (int k0 = 0; k0 < ke; k0 += 4) {
           // bordered: MFMA steps k0 < NC only; the step k0 = NC carries the border terms
           const bool mstep = !BRD || k0 < NC;
@@ -603,18 +612,18 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a) {
           tr[u] = floatx4{0.f, 0.f, 0.f, 0.f};
           ti[u] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
-        lds_gemm<BPW, 0>(sL, a.op_pitch, sS, P, trow, tcol, lr, lg, ke, tr, ti);
+        lds_gemm<BPW, 0, KS>(sL, a.op_pitch, sS, P, trow, tcol, lr, lg, ke, tr, ti);
         put_t(sT);
         __syncthreads();
         const float2* R = sL + (a.rops ? a.n_dense * slot : 0);
         int kk = 0;
         for (; kk + 1 < a.n_dense; ++kk) {
-          lds_gemm_pair<BPW>(kk & 1 ? sT1 : sT, P, R + kk * slot, sL + (kk + 1) * slot, a.op_pitch, sS, P, trow, tcol, lr,
+          lds_gemm_pair<BPW, KS>(kk & 1 ? sT1 : sT, P, R + kk * slot, sL + (kk + 1) * slot, a.op_pitch, sS, P, trow, tcol, lr,
                              lg, ke, cr, ci, tr, ti);
           put_t(kk & 1 ? sT : sT1);
           __syncthreads();
         }
-        lds_gemm<BPW, 2>(kk & 1 ? sT1 : sT, P, R + kk * slot, a.op_pitch, trow, tcol, lr, lg, ke, cr, ci);
+        lds_gemm<BPW, 2, KS>(kk & 1 ? sT1 : sT, P, R + kk * slot, a.op_pitch, trow, tcol, lr, lg, ke, cr, ci);
       }
       // C += i sum_k (L_k S) R_k^dag, every factor staged through LDS (sL) so the fragment
       // loops are the same pipelined LDS reads as the H_eff products.
@@ -629,7 +638,7 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a) {
           tr[u] = floatx4{0.f, 0.f, 0.f, 0.f};
           ti[u] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
-        lds_gemm<BPW, 0>(sL, P, sS, P, trow, tcol, lr, lg, ke, tr, ti);    // T = L S
+        lds_gemm<BPW, 0, KS>(sL, P, sS, P, trow, tcol, lr, lg, ke, tr, ti);    // T = L S
 #pragma unroll
         for (int u = 0; u < BPW; ++u) {
           if (!tval[u]) continue;
@@ -642,7 +651,7 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a) {
           stage_operator<NP, P, T>(sL, a.rops + ((size_t)set * a.n_dense + kk) * nn, n, tid);
         }
         __syncthreads();
-        lds_gemm<BPW, 2>(sT, P, sL, P, trow, tcol, lr, lg, ke, cr, ci);    // C += i T R^dag
+        lds_gemm<BPW, 2, KS>(sT, P, sL, P, trow, tcol, lr, lg, ke, cr, ci);    // C += i T R^dag
       }
       // k = -i C + D o S, formed in place: afterwards kr = ci, ki = -cr.
       if (!DFOLD && has_d) {
@@ -906,17 +915,24 @@ lindblad_rk4_resident(ResidentArgs a) {
   resident_body<NB, W, BPW, MINW, DENSE, REC, BRD, DB, false, false>(a);
 }
 
-// dense jump operators resident in LDS
-template <int NB, int W, int BPW, int MINW, bool REC>
+// no dense jump operators, the reduction's length built in
+template <int NB, int W, int BPW, int MINW, bool REC, int KS>
 __global__ void __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(MINW)))
-lindblad_rk4_resident_ops(ResidentArgs a) {
-  resident_body<NB, W, BPW, MINW, true, REC, false, false, false, true>(a);
+lindblad_rk4_resident_plain(ResidentArgs a) {
+  resident_body<NB, W, BPW, MINW, false, REC, false, true, false, false, KS>(a);
 }
 
-template <int NB, int W, int BPW, int MINW, bool DENSE, bool BRD, bool DB, bool RES>
+// dense jump operators, resident in LDS (RES) or staged
+template <int NB, int W, int BPW, int MINW, bool REC, bool RES, int KS>
 __global__ void __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(MINW)))
+lindblad_rk4_resident_ops(ResidentArgs a) {
+  resident_body<NB, W, BPW, MINW, true, REC, false, false, false, RES, KS>(a);
+}
+
+template <int NB, int W, int BPW, int MINW, bool DENSE, bool BRD, bool DB, bool RES, int KS = 0>
+__global__ void __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(KS > 0 && W < 16 ? 3 : MINW)))
 lindblad_rk4_resident_driven(ResidentArgs a) {
-  resident_body<NB, W, BPW, MINW, DENSE, true, BRD, DB, true, RES>(a);
+  resident_body<NB, W, BPW, MINW, DENSE, true, BRD, DB, true, RES, KS>(a);
 }
 
 // ------------------------------------------------------------------------ host launch
@@ -957,27 +973,72 @@ hipError_t launch_kernel(void (*k)(ResidentArgs), const ResidentArgs& a, int wav
   return hipGetLastError();
 }
 
+// the k-steps of the reductions that are built in: sizes from 16 (NB - 1) + 5 (index 0) or + 1 (-1) on;
+// lindblad_edge.hip takes most of the latter with dense operators
+template <int NB, int I>
+constexpr int k_steps() { return 4 * (NB - 1) + 2 + I; }
+
+template <int NB, int W, int BPW, int MINW, bool RES, int KS>
+hipError_t launch_ops(const ResidentArgs& a, size_t lds, hipStream_t stream) {
+  const bool rec = a.nout > 0 && (a.obs != nullptr || a.states != nullptr);
+  if (a.heff_step > 0)
+    return launch_kernel(lindblad_rk4_resident_driven<NB, W, BPW, MINW, true, false, false, RES, KS>, a, W, lds, stream);
+  return rec ? launch_kernel(lindblad_rk4_resident_ops<NB, W, BPW, MINW, true, RES, KS>, a, W, lds, stream)
+             : launch_kernel(lindblad_rk4_resident_ops<NB, W, BPW, MINW, false, RES, KS>, a, W, lds, stream);
+}
+
+template <int NB, int W, int BPW, int MINW, bool RES>
+hipError_t launch_dense(const ResidentArgs& a, size_t lds, hipStream_t stream) {
+  if constexpr (NB >= 2 && !(NB == 4 && RES)) {   // the 16 waves of NB = 4 leave 128 VGPRs: resident, it spills
+    switch (cdiv(a.n, 4)) {
+      case k_steps<NB, 0>(): return launch_ops<NB, W, BPW, MINW, RES, k_steps<NB, 0>()>(a, lds, stream);
+      case k_steps<NB, 1>(): return launch_ops<NB, W, BPW, MINW, RES, k_steps<NB, 1>()>(a, lds, stream);
+      case k_steps<NB, 2>(): return launch_ops<NB, W, BPW, MINW, RES, k_steps<NB, 2>()>(a, lds, stream);
+      case k_steps<NB, -1>():
+        if constexpr (NB == 4) return launch_ops<NB, W, BPW, MINW, RES, k_steps<NB, -1>()>(a, lds, stream);
+    }
+  }
+  return launch_ops<NB, W, BPW, MINW, RES, 0>(a, lds, stream);
+}
+
+template <int NB, int W, int BPW, int MINW, int KS>
+hipError_t launch_plain(const ResidentArgs& a, size_t lds, hipStream_t stream) {
+  const bool rec = a.nout > 0 && (a.obs != nullptr || a.states != nullptr);
+  if (rec) return launch_kernel(lindblad_rk4_resident_plain<NB, W, BPW, MINW, true, KS>, a, W, lds, stream);
+  // two tiles a wave, unrolled by 2: without records the remainder of an odd length spills a register
+  if constexpr (BPW == 2 && KS % 2 == 1)
+    return launch_kernel(lindblad_rk4_resident<NB, W, BPW, MINW, false, false, false, true>, a, W, lds, stream);
+  else
+    return launch_kernel(lindblad_rk4_resident_plain<NB, W, BPW, MINW, false, KS>, a, W, lds, stream);
+}
+
 template <int NB, int W, int BPW, int MINW, bool DENSE, bool BRD, bool DB>
 hipError_t launch_rec2(const ResidentArgs& a, size_t lds, hipStream_t stream) {
   const bool rec = a.nout > 0 && (a.obs != nullptr || a.states != nullptr);
+  if constexpr (DENSE && BPW == 1) {
+    static_assert(MINW <= 5, "the budget of the driven kernels");
+    return a.op_pitch > 0 ? launch_dense<NB, W, BPW, MINW, true>(a, lds, stream)
+                          : launch_dense<NB, W, BPW, MINW, false>(a, lds, stream);
+  }
+  if constexpr (!DENSE && (BPW == 1 || NB == 5) && !BRD && DB && NB >= 2) {
+    if (a.heff_step <= 0) {
+      switch (cdiv(a.n, 4)) {
+        case k_steps<NB, -1>(): return launch_plain<NB, W, BPW, MINW, k_steps<NB, -1>()>(a, lds, stream);
+        case k_steps<NB, 0>(): return launch_plain<NB, W, BPW, MINW, k_steps<NB, 0>()>(a, lds, stream);
+        case k_steps<NB, 1>(): return launch_plain<NB, W, BPW, MINW, k_steps<NB, 1>()>(a, lds, stream);
+        case k_steps<NB, 2>(): return launch_plain<NB, W, BPW, MINW, k_steps<NB, 2>()>(a, lds, stream);
+      }
+    }
+  }
   if (a.heff_step > 0) {
     // driven systems run the default shape; at 6 waves per SIMD the step's extra addresses spill
     // two registers, and the few operators of a driven call do not need the occupancy
     constexpr Shape first = (BRD ? kBorderShapes : kShapes)[NB][0];
     constexpr int MW = MINW > 5 ? 5 : MINW;
     if constexpr (W == first.w && BPW == first.bpw) {
-      if constexpr (DENSE && BPW == 1) {
-        if (a.op_pitch > 0)
-          return launch_kernel(lindblad_rk4_resident_driven<NB, W, BPW, MW, DENSE, BRD, DB, true>, a, W, lds, stream);
-      }
       return launch_kernel(lindblad_rk4_resident_driven<NB, W, BPW, MW, DENSE, BRD, DB, false>, a, W, lds, stream);
     }
     return hipErrorInvalidValue;
-  }
-  if constexpr (DENSE && BPW == 1) {
-    if (a.op_pitch > 0)
-      return rec ? launch_kernel(lindblad_rk4_resident_ops<NB, W, BPW, MINW, true>, a, W, lds, stream)
-                 : launch_kernel(lindblad_rk4_resident_ops<NB, W, BPW, MINW, false>, a, W, lds, stream);
   }
   return rec ? launch_kernel(lindblad_rk4_resident<NB, W, BPW, MINW, DENSE, true, BRD, DB>, a, W, lds, stream)
              : launch_kernel(lindblad_rk4_resident<NB, W, BPW, MINW, DENSE, false, BRD, DB>, a, W, lds, stream);
@@ -1030,8 +1091,9 @@ size_t lds_layout(int n, int variant, int n_dense, int n_eops, int nbuf);
 // or 0 to stage them.  They are resident when the workgroups that the batch puts on a CU still
 // fit with them, so the occupancy of a large batch is never given up; shapes with one tile per
 // wave only (with two the shared loop spills).  us per RK4 step, staged / resident, one operator:
-// n = 8, 16 jump operators 56.6 / 35.9; n = 24, 4 sandwich terms 44 / 26, 16 jump operators 127 /
-// 85; n = 32, 4 45 / 33; n = 48, 4 120 / 106; n = 64, 1 75.4 / 74.9; 256 operators n = 32, 4 48 / 37.
+// n = 24, 4 sandwich terms 44 / 26, 16 jump operators 127 / 85; n = 32, 4 45 / 33; n = 48, 4 120 / 106;
+// n = 64, 1 75.4 / 74.9; 256 operators n = 32, 4 48 / 37 (reductions of run-time length on both sides; built
+// in: n = 28 with 8 sandwich terms, resident, 39, n = 30, where they no longer fit, staged, 85).
 // The second T buffer takes the place of the staging buffer of the staged layout.
 int operand_pitch(int n) { return ((n + 3) & ~3) + 1; }
 size_t dense_lds_bytes(int n, int n_dense, bool rops) {
