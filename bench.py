@@ -686,7 +686,8 @@ def bench_ragged(args):
     out = _base(f"RK4 rho-steps/s (uneven batch n in 16..256, {args.precision})", value, args,
                 total_ms / args.steps, _dtype(args.precision),
                 "synthetic (seeded GUE instances, on-site dephasing + 4 dense L_k)", config,
-                _roofline("lindblad_ragged_persistent" if persistent else shape, tflops,
+                _roofline(shape if not persistent else "lindblad_ragged_persistent" if rb.variant < rb.variants()
+                          else "lindblad_ragged_left + lindblad_ragged_stage", tflops,
                           float(np.mean(per)), args.precision))
     if not args.no_check:
         from oracle import lindblad as ol
