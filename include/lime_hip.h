@@ -269,8 +269,9 @@ int lime_adjoint_seed(int32_t batch, int32_t n, int32_t flags, void* lam, const 
  *   eops   [n_e][m], obs [nsteps][rows][n_e]: obs = sum_j eops_ej x_j of every stored state,
  *          or both NULL
  *   work   lime_linear_rk4_workspace_bytes(m) bytes of device memory
- * The step's increment is formed once (RK4 of a constant G is a polynomial of G) and steps are
- * taken in blocks, so records differ from step-by-step RK4 by FP64 rounding.
+ * The step's matrix is formed once (RK4 of a constant G is a polynomial of G), to 106 bits, and steps are
+ * taken in blocks: a record differs from step-by-step RK4 by FP64 rounding of its own size, also
+ * where the system decays.
  * Replaces lime's _redfield (lime/oqs.py:373-472) and the loop of phys.expm (phys.py:1352-1401).
  */
 int lime_linear_rk4(int32_t m, int32_t rows, int32_t nsteps, double dt, const void* g, void* x, void* states,
