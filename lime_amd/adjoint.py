@@ -143,7 +143,7 @@ class ChainQRT:
         B, n, h = self.B, self.n, self.dt
         dev = self.dev
         mu_h = self.mu.conj().transpose(0, 1).contiguous()
-        Gt = G.to(dev, torch.complex128).t().contiguous()     # (Nt, B): Gt[k] contiguous
+        Gt = G.to(dev, torch.complex128).resolve_conj().t().contiguous()     # (Nt, B): Gt[k] contiguous
         lam = torch.zeros((B, n, n), dtype=torch.complex128, device=dev)
         outa = torch.zeros((B, n), dtype=torch.complex128, device=dev)
         outb = torch.zeros((B, n), dtype=torch.complex128, device=dev)

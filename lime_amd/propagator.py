@@ -32,7 +32,8 @@ def device():
 def as_c128(x, dev):
     """Array-like or tensor -> contiguous complex128 tensor on ``dev``."""
     if isinstance(x, torch.Tensor):
-        t = x.to(device=dev, dtype=torch.complex128)
+        # a conjugate view's memory holds the unconjugated numbers, and the kernels read the memory
+        t = x.to(device=dev, dtype=torch.complex128).resolve_conj().resolve_neg()
     else:
         if hasattr(x, "toarray"):          # scipy.sparse
             x = x.toarray()
@@ -45,7 +46,7 @@ def _check(t, what, shape, dtype, dev):
     sizes alone: its shape, dtype, layout and device are checked here, on the host."""
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{what} must be a torch tensor")
-    if t.dtype != dtype or not t.is_contiguous() or t.device != dev:
+    if t.dtype != dtype or not t.is_contiguous() or t.device != dev or t.is_conj() or t.is_neg():
         raise ValueError(f"{what} must be a contiguous {dtype} tensor on {dev}")
     if tuple(t.shape) != tuple(shape):
         raise ValueError(f"{what} has shape {tuple(t.shape)}, expected {tuple(shape)}")
@@ -293,10 +294,10 @@ class LindbladPropagator:
         adj._work = None
         adj.variant = self._tile_variant()
         adj.force_tiled = True
-        h = lambda t: t.conj().transpose(-1, -2).contiguous()
+        h = lambda t: t.conj().transpose(-1, -2).resolve_conj().contiguous()
         adj.heff = (-h(self.heff)).contiguous()
         adj.heff_c128 = (-h(self.heff_c128)).contiguous()
-        adj.dmat = self.dmat.conj().contiguous() if self.dmat is not None else None
+        adj.dmat = self.dmat.conj().resolve_conj().contiguous() if self.dmat is not None else None
         adj.lops = h(self.lops) if self.lops is not None else None
         # R = L (rops None) stays implicit: the adjoint's right factors are adj.lops too
         adj.rops = h(self.rops) if self.rops is not None else None
