@@ -32,7 +32,7 @@ from scipy.linalg import eigh
 from . import _lib
 from . import superoperator as so
 from .mol import Result
-from .propagator import LindbladPropagator, as_c128, device
+from .propagator import LindbladPropagator, _check, as_c128, device
 
 
 def _dense(a):
@@ -93,21 +93,37 @@ def _column_chunk(M, budget=1 << 28):
     return max(1, budget // (M * M * 16))
 
 
-def linear_rk4(G, x, dt, nsteps, eops=None, keep=True):
-    """``nsteps`` RK4 steps of dx/dt = G x (``lime_linear_rk4``, FP64) for the rows of ``x``
-    (rows, M), a complex128 tensor on the GPU.
-
-    Returns (the final rows, the rows after every step (nsteps, rows, M) or None without
-    ``keep``, sum_j eops[e, j] x_j after every step (nsteps, rows, n_e) or None)."""
-    dev = x.device
-    lib = _lib.load()
-    rows, M = x.shape
+def _linear_operands(G, x, eops):
+    """(G, a copy of x, eops) as ``lime_linear_rk4`` reads them: row-major complex128 on x's device."""
+    if not isinstance(x, torch.Tensor) or x.dim() != 2:
+        raise ValueError("x must be a tensor (rows, M)")
+    dev, M = x.device, x.shape[1]
     Gt = as_c128(G, dev)
     if Gt.shape != (M, M):
         raise ValueError(f"the generator has shape {tuple(Gt.shape)}, expected ({M}, {M})")
-    if eops is not None and tuple(eops.shape[1:]) != (M,):
-        raise ValueError(f"observables have shape {tuple(eops.shape)}, expected (n_e, {M})")
-    x = x.clone()
+    x = x.to(torch.complex128).clone(memory_format=torch.contiguous_format)
+    if eops is not None:
+        eops = as_c128(eops, dev)
+        if eops.dim() != 2 or eops.shape[1] != M:
+            raise ValueError(f"observables have shape {tuple(eops.shape)}, expected (n_e, {M})")
+        _check(eops, "eops", eops.shape, torch.complex128, dev)
+    _check(Gt, "G", (M, M), torch.complex128, dev)
+    _check(x, "x", x.shape, torch.complex128, dev)
+    return Gt, x, eops
+
+
+def linear_rk4(G, x, dt, nsteps, eops=None, keep=True):
+    """``nsteps`` RK4 steps of dx/dt = G x (``lime_linear_rk4``, FP64) for the rows of ``x``
+    (rows, M), a tensor on the GPU (not changed).
+
+    Returns (the final rows, the rows after every step (nsteps, rows, M) or None without
+    ``keep``, sum_j eops[e, j] x_j after every step (nsteps, rows, n_e) or None), complex128."""
+    Gt, x, eops = _linear_operands(G, x, eops)
+    dev = x.device
+    if dev.type != "cuda":
+        raise ValueError(f"x must be on the GPU, not on {dev}")
+    lib = _lib.load()
+    rows, M = x.shape
     n_e = 0 if eops is None else eops.shape[0]
     empty = lambda *shape: torch.empty(shape, dtype=torch.complex128, device=dev)
     obs = empty(nsteps, rows, n_e) if n_e else None
