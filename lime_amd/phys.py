@@ -99,13 +99,28 @@ def ldo(b, A):
     return A @ b
 
 
+def _steps_in_blocks(M, steps):
+    """Does ``expm`` in FP64 run on ``lime_linear_rk4`` (blocks of steps) for M x M matrices, or step by
+    step on the one-sided per-stage kernels?
+
+    All M rows of U are stepped, so the products are M x M x M, which the per-stage kernels stage
+    through LDS and ``lime_linear_rk4``, made for few rows, does not (38 against 75 TFLOP/s at
+    M = 2048).  It pays by its fewer launches and products while M is small, above that once many steps
+    share the block's matrix.  us, one call in blocks / step by step: M = 128, 64 steps 170 / 2317,
+    M = 320, 1 step 72 / 86; M = 384, 8 steps 731 / 615, 20 steps 1137 / 1522; M = 512, 8 steps 1317 / 785, 20
+    steps 1825 / 1927, 64 steps 3927 / 6109; M = 640, 20 steps 3921 / 3383; M = 1024, 8 steps 9919 / 3814; M = 4096,
+    1 step 57900 / 28700."""
+    return M <= 320 or (M <= 512 and steps >= 20)
+
+
 def expm(A, t, method="EOM", precision="fp64"):
     """U(t_k) = e^{A t_k} for the times t (phys.py:1352-1401), as lime's list of Nt arrays.
 
     'EOM': U(t_0) = I and each further entry one RK4 step of dU/dt = A U with
     dt = t[1] - t[0] (lime's ``interval``), i.e. U(t_k) = P(dt A)^k with the RK4 polynomial
-    P; the Nt - 1 steps run on ``lime_linear_rk4`` in FP64 (the default), else on the
-    one-sided per-stage kernels, recording every step.  'SOS' raises NotImplementedError, as in lime.
+    P; the Nt - 1 steps run on ``lime_linear_rk4`` in FP64 (the default) where
+    ``_steps_in_blocks``, else on the one-sided per-stage kernels, recording every step.
+    'SOS' raises NotImplementedError, as in lime.
     """
     if method == "SOS":
         raise NotImplementedError("Method of SOS has not been implemented. Choose from EOM")
@@ -116,11 +131,12 @@ def expm(A, t, method="EOM", precision="fp64"):
     from .redfield import _column_chunk, _dense, linear_rk4, liouville_propagator
     t = np.asarray(t, dtype=np.float64)
     Nt = len(t)
-    if precision == "fp64":
+    A = _dense(A)
+    if A.ndim != 2 or A.shape[0] != A.shape[1]:
+        raise ValueError(f"A must be (M, M), got {A.shape}")
+    if precision == "fp64" and _steps_in_blocks(A.shape[0], Nt - 1):
         from .propagator import as_c128, device
-        At = as_c128(_dense(A), device())
-        if At.dim() != 2 or At.shape[0] != At.shape[1]:
-            raise ValueError(f"A must be (M, M), got {tuple(At.shape)}")
+        At = as_c128(A, device())
         M = At.shape[0]
         At = At.transpose(0, 1).contiguous()       # the rows of U step with A^T: U_k = U_(k-1) P(dt A)
         x = torch.eye(M, dtype=torch.complex128, device=At.device)
