@@ -132,6 +132,8 @@ def expm(A, t, method="EOM", precision="fp64"):
     t = np.asarray(t, dtype=np.float64)
     Nt = len(t)
     A = _dense(A)
+    if A.ndim == 3 and A.shape[0] == 1:
+        A = A[0]
     if A.ndim != 2 or A.shape[0] != A.shape[1]:
         raise ValueError(f"A must be (M, M), got {A.shape}")
     if precision == "fp64" and _steps_in_blocks(A.shape[0], Nt - 1):

@@ -99,6 +99,8 @@ def _linear_operands(G, x, eops):
         raise ValueError("x must be a tensor (rows, M)")
     dev, M = x.device, x.shape[1]
     Gt = as_c128(G, dev)
+    if Gt.dim() == 3 and Gt.shape[0] == 1:
+        Gt = Gt[0]
     if Gt.shape != (M, M):
         raise ValueError(f"the generator has shape {tuple(Gt.shape)}, expected ({M}, {M})")
     x = x.to(torch.complex128).clone(memory_format=torch.contiguous_format)

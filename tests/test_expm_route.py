@@ -25,9 +25,19 @@ def test_both_routes_step_rk4(M, steps):
         k3 = A @ (X + h / 2 * k2)
         X = X + h / 6 * (k1 + 2 * k2 + 2 * k3 + A @ (X + h * k3))
         ref.append(X)
-    U = phys.expm(A, h * np.arange(steps + 1))
-    assert len(U) == steps + 1 and all(u.shape == (M, M) for u in U)
-    assert max(np.abs(u - r).max() for u, r in zip(U, ref)) < 1e-13 * max(1.0, np.abs(ref[-1]).max())
+    for form in (A, A[None]):
+        U = phys.expm(form, h * np.arange(steps + 1))
+        assert len(U) == steps + 1 and all(u.shape == (M, M) for u in U)
+        assert max(np.abs(u - r).max() for u, r in zip(U, ref)) < 1e-13 * max(1.0, np.abs(ref[-1]).max())
+
+
+@pytest.mark.gpu
+def test_redfield_takes_a_tensor_with_a_leading_set():
+    from lime_amd.oqs import _redfield
+    rng = np.random.default_rng(1)
+    R, rho = 0.1 * rng.standard_normal((9, 9)) + 0j, np.diag([0.5, 0.3, 0.2]) + 0j
+    a, b = (_redfield(r, rho, Nt=3, dt=0.1) for r in (R, R[None]))
+    assert np.array_equal(np.array(a.rholist), np.array(b.rholist))
 
 
 def test_what_is_no_square_matrix_is_refused():
