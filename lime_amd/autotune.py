@@ -9,6 +9,7 @@ HIP events on the launch stream), keeps the fastest, and caches the choice per
 (``LIME_TUNE_CACHE``, else ``$XDG_CACHE_HOME/lime_amd/tune.json`` or
 ``~/.cache/lime_amd/tune.json``; never inside the package).
 """
+import hashlib
 import json
 import os
 import sys
@@ -116,13 +117,22 @@ def tune(prop, rho, dt, steps=4, n_eops=0, force=False, verbose=False, eops_t=No
     return best, times
 
 
+def ragged_key(rb):
+    """One choice per batch shape: the instances' (n, K_d), in any order (batches of one sum of
+    n^3 (1 + K_d) differ 4x in what the persistent launch and the launches per phase take), and the
+    cap on persistent workgroups, which leaves only the persistent launch."""
+    shape = ",".join(f"{n}x{k}" for n, k in sorted(zip(map(int, rb.sizes), map(int, rb.kd))))
+    return (f"{_version()}:ragged:c{rb.count}:s{hashlib.sha256(shape.encode()).hexdigest()[:16]}"
+            f":g{rb.max_groups}")
+
+
 def tune_ragged(rb, dt, steps=2, force=False, verbose=False):
-    """Pick the fastest persistent launch shape of a ``RaggedLindblad`` batch (states are
-    restored afterwards); cached per (instance count, sum of n^3 (1 + K_d))."""
-    key = f"{_version()}:ragged:c{rb.count}:w{int(rb.work_units)}"
+    """Pick the fastest of a ``RaggedLindblad`` batch's launches (states are restored
+    afterwards); cached per ``ragged_key``."""
+    key = ragged_key(rb)
     with _lock:
         cache = _load()
-        if not force and key in cache:
+        if not force and key in cache and 0 <= int(cache[key]["variant"]) < rb.launches():
             rb.variant = int(cache[key]["variant"])
             return rb.variant, cache[key].get("ms", {})
     saved = rb.rho.clone()
