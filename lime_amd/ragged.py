@@ -191,7 +191,7 @@ class RaggedLindblad:
         p = _lib.StepParams()
         p.dt, p.nsteps = float(dt), int(nsteps)
         s = stream if stream is not None else torch.cuda.current_stream(self.dev)
-        if tiled >= 0:
+        if 0 <= tiled < self.launches() - self.variants():     # what is not offered the library refuses
             tiles = self._tile_lists(TILE_EDGES[tiled])
             _lib.check(self._lib.lime_lindblad_rk4_ragged_tiles(ctypes.byref(r), ctypes.byref(tiles),
                                                                 ctypes.byref(p), ctypes.c_void_p(s.cuda_stream)))

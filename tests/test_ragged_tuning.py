@@ -103,3 +103,19 @@ def test_uncapped_then_capped_and_the_reverse(tmp_path, monkeypatch):
             assert 0 <= rb.variant < rb.launches()
         assert len(autotune._cache) == 2
         assert all(len(v["ms"]) == (5 if k.endswith(":g1") else 7) for k, v in autotune._cache.items())
+
+
+@pytest.mark.parametrize("variant,max_groups", [(-1, 0), (7, 0), (8, 0), (5, 1), (6, 3)])
+def test_a_launch_that_is_not_offered_is_refused(variant, max_groups):
+    """By the library, before any GPU work: the sizes are checked first."""
+    from types import SimpleNamespace
+
+    from lime_amd import _lib
+    from lime_amd.ragged import RaggedLindblad
+    rb = object.__new__(RaggedLindblad)
+    rb._lib = _lib.load()
+    rb.count, rb.variant, rb.max_groups = 1, variant, max_groups
+    rb.inst = rb.order = rb.ops = rb.rho = rb.work = rb.queue = torch.zeros(1)
+    rb.sizes, rb.kd, rb.cost, rb._lists, rb.dev = np.array([4]), np.array([0]), np.array([64.0]), {}, "cpu"
+    with pytest.raises(_lib.LimeError, match="variant"):
+        rb.step(0.01, 1, stream=SimpleNamespace(cuda_stream=0))
