@@ -5,6 +5,7 @@
 Cross-compiles without a GPU.  Packed-FP32 instructions are disabled on every HIP
 translation unit (``-Xclang -target-feature -Xclang -packed-fp32-ops``).
 """
+import hashlib
 import os
 import subprocess
 import sys
@@ -31,8 +32,20 @@ def sources():
     return sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".hip"))
 
 
+def build_id(extra=()):
+    """What the library is built from: a hash of the sources, headers and flags.  Part of
+    ``lime_version``, so that launch choices tuned on one build are not taken over by another."""
+    h = hashlib.sha256(" ".join([ARCH, *FLAGS[:FLAGS.index("-I")], *extra]).encode())
+    for folder in (CSRC, INCLUDE):
+        for name in sorted(f for f in os.listdir(folder) if f.endswith((".hip", ".hpp", ".h"))):
+            with open(os.path.join(folder, name), "rb") as f:
+                h.update(name.encode() + b"\0" + f.read() + b"\0")
+    return h.hexdigest()[:12]
+
+
 def _compile(src, extra):
     obj = os.path.join(OBJDIR, os.path.basename(src)[:-4] + ".o")
+    extra = [*extra, f'-DLIME_BUILD_ID="{build_id(extra)}"'] if os.path.basename(src) == "abi.hip" else extra
     cmd = [HIPCC, *FLAGS, *extra, "-c", src, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:

@@ -219,7 +219,12 @@ extern "C" {
 
 const char* lime_last_error(void) { return g_last_error.c_str(); }
 
-const char* lime_version(void) { return "lime_hip 0.3 (gfx950)"; }
+// with a hash of what the library was built from (the build passes it): tuned launch choices are kept
+// per build
+#ifndef LIME_BUILD_ID
+#define LIME_BUILD_ID "unknown"
+#endif
+const char* lime_version(void) { return "lime_hip 0.3 (gfx950) build " LIME_BUILD_ID; }
 
 int lime_lindblad_max_n(int32_t n_dense, int32_t flags) {
   if ((flags & LIME_F_PREC_MASK) != LIME_F_PREC_FP32) return 0;
