@@ -83,6 +83,29 @@ def as_c128_stack(xs, dev, dim=0):
     return torch.stack([as_c128(x, dev) for x in xs], dim=dim)
 
 
+#: operators are looked at on the GPU this many bytes at a time (at least one operator)
+_STACK_BYTES = 64 << 20
+
+
+def _is_diagonal(t):
+    """Are all off-diagonal entries of (sets, n, n) exactly zero and the diagonals finite?  (NumPy)"""
+    d = np.diagonal(t, axis1=-2, axis2=-1)
+    if not np.all(np.isfinite(d)):
+        return False
+    step = max(1, (1 << 14) // max(1, t.shape[-1]))
+    return all(np.count_nonzero(t[:, r:r + step]) == np.count_nonzero(d[:, r:r + step])
+               for r in range(0, t.shape[-1], step))
+
+
+def _look(T):
+    """The diagonals of a stack of operators (sets, K, n, n) and, per operator, whether it has an
+    off-diagonal entry or a diagonal one that is not finite."""
+    d = torch.diagonal(T, dim1=-2, dim2=-1).clone()
+    nz = T != 0
+    torch.diagonal(nz, dim1=-2, dim2=-1).copy_((d - d) != 0)
+    return d, torch.any(nz.transpose(0, 1).reshape(T.shape[1], -1), dim=1)
+
+
 def fold_jump_operators(H, c_ops, dev=None):
     """Split jump operators into H_eff, the Hadamard dissipator D and dense operators.
 
@@ -91,10 +114,10 @@ def fold_jump_operators(H, c_ops, dev=None):
     lops (S,Kd,N,N) or None.  A jump operator is *diagonal* when every off-diagonal
     entry of every set is exactly zero and its diagonal is finite.
 
-    Host operators are looked at on the host, operators on the GPU with one read-back for all
-    of them; of the diagonal ones only the diagonals go to the GPU.  (A product, a test and a
-    synchronisation per operator took 110 us each: 3.4 of 5.0 ms of a two-time correlation
-    with 16 on-site operators.)
+    Host operators are looked at on the host, operators on the GPU in stacks of up to ``_STACK_BYTES`` with
+    one read-back for all of them; of the diagonal ones only the diagonals are kept, so many of them cost
+    no memory.  (A product, a test and a synchronisation per
+    operator took 110 us each: 3.4 of 5.0 ms of a two-time correlation with 16 on-site operators.)
     """
     dev = dev or device()
     Ht = as_c128(H, dev)
@@ -103,48 +126,64 @@ def fold_jump_operators(H, c_ops, dev=None):
     if Ht.dim() != 3 or Ht.shape[-1] != Ht.shape[-2]:
         raise ValueError(f"H must be (N, N) or (S, N, N), got {tuple(Ht.shape)}")
     S, n = Ht.shape[0], Ht.shape[-1]
-    ops = []                                   # each (1 or S, n, n), NumPy or on a GPU
+    ops, diag = {}, {}                         # dense (or not looked at yet), and diagonals, by number
     groups = {}                                # GPU operators by their number of sets
-    for k, c in enumerate(c_ops or []):
+    c_ops = list(c_ops or [])
+
+    def take(k, c):
         t = _on_host(c)
-        t = c.to(device=dev, dtype=torch.complex128) if t is None else t
+        t = c if t is None else t
         t = t[None] if t.ndim == 2 else t
         if tuple(t.shape[-2:]) != (n, n):
             raise ValueError(f"c_ops[{k}] has shape {tuple(t.shape)}, expected (..., {n}, {n})")
-        if t.ndim != 3 or t.shape[0] not in (1, S):
-            raise ValueError(f"c_ops[{k}] has {t.shape[0]} sets, expected {S}")
-        ops.append(t)
+        sets = t.shape[0]
+        if t.ndim != 3 or sets not in (1, S):
+            raise ValueError(f"c_ops[{k}] has {sets} sets, expected {S}")
         if isinstance(t, torch.Tensor):
-            groups.setdefault(t.shape[0], []).append(k)
-    off, diag, stacks = {}, {}, {}
+            ops[k] = t
+            groups.setdefault(sets, []).append(k)
+        elif not _is_diagonal(t):
+            ops[k] = t
+        else:
+            diag[k] = np.diagonal(t, axis1=-2, axis2=-1).copy()
+
+    for k, c in enumerate(c_ops):
+        take(k, c)
+    looked, stacks = [], {}
     for sets, ks in groups.items():
-        T = torch.stack([ops[k] for k in ks], dim=1)        # (sets, K, n, n)
-        d = torch.diagonal(T, dim1=-2, dim2=-1)
-        nz = T != 0
-        torch.diagonal(nz, dim1=-2, dim2=-1).copy_((d - d) != 0)     # a diagonal entry that is not finite
-        stacks[sets] = (T, torch.any(nz.transpose(0, 1).reshape(len(ks), -1), dim=1))
-        diag.update({k: d[:, x] for x, k in enumerate(ks)})
-    if groups:
-        off = dict(zip([k for ks in groups.values() for k in ks],
-                       torch.cat([x for _, x in stacks.values()]).tolist()))
-    for k, t in enumerate(ops):
-        if k not in off:
-            diag[k] = np.diagonal(t, axis1=-2, axis2=-1)
-            off[k] = np.count_nonzero(t) - np.count_nonzero(diag[k]) + np.count_nonzero(~np.isfinite(diag[k]))
-    diags = [diag[k] for k in range(len(ops)) if not off[k]]
-    dense = [k for k in range(len(ops)) if off[k]]
+        many = max(1, _STACK_BYTES // max(1, 16 * sets * n * n))
+        for part in (ks[x:x + many] for x in range(0, len(ks), many)):
+            T = torch.stack([ops[k].to(device=dev, dtype=torch.complex128) for k in part], dim=1)   # (sets, K, n, n)
+            d, off = _look(T)
+            looked.append((part, d, off))
+            if len(part) == len(ks):
+                stacks[tuple(ks)] = T
+            del T                                           # before the next stack is made
+    if looked:
+        off = torch.cat([x for _, _, x in looked]).tolist()
+        for part, d, _ in looked:
+            diag.update({k: d[:, x] for x, k in enumerate(part) if not off[x]})
+            del off[:len(part)]
+    diags = [diag[k] for k in sorted(diag)]
+    dense = [k for k in sorted(ops) if k not in diag]
+    stacks = {ks: T for ks, T in stacks.items() if list(ks) == dense}
     gamma = torch.zeros_like(Ht)
     dmat = lops = None
 
     def stack(xs):                                          # (1 or S, K, ...)
         sets = max(x.shape[0] for x in xs)
+        mixed = len({isinstance(x, torch.Tensor) for x in xs}) > 1
+        if mixed or 16 * sets * len(xs) * int(np.prod(xs[0].shape[1:])) > _STACK_BYTES:
+            out = torch.empty((sets, len(xs), *xs[0].shape[1:]), dtype=torch.complex128, device=dev)
+            for k, x in enumerate(xs):
+                out[:, k] = x if isinstance(x, torch.Tensor) else torch.as_tensor(x)
+            return out
         wide = [x.expand(sets, *x.shape[1:]) if isinstance(x, torch.Tensor) else
                 np.broadcast_to(x, (sets, *x.shape[1:])) for x in xs]
         return as_c128_stack(wide, dev, dim=1)
 
     if dense:
-        whole = next((stacks[x][0] for x, ks in groups.items() if ks == dense), None)
-        L = stack([ops[k] for k in dense]) if whole is None else whole
+        L = stacks[tuple(dense)] if stacks else stack([ops[k] for k in dense])
         if n <= 64:                                         # one launch: sum L^dag L = V^dag V
             V = L.reshape(L.shape[0], -1, n)
             gamma = gamma + torch.matmul(V.conj().transpose(-1, -2), V)
