@@ -85,16 +85,23 @@ def as_c128_stack(xs, dev, dim=0):
 
 #: operators are looked at on the GPU this many bytes at a time (at least one operator)
 _STACK_BYTES = 64 << 20
+#: host operators of this size go to the GPU one by one, smaller ones stacked on the host: a copy costs
+#: 25 us, a stack 0.25 us a KB (16 of n = 512: 4.9 / 9.5 ms)
+_COPY_BYTES = 256 << 10
+#: host operators of this size are looked at on the GPU, past their first rows: the host reads 11 GB/s, the
+#: copies take 20 (32 diagonal ones of n = 1024: 49 ms on the host, 25 on the GPU)
+_LOOK_BYTES = 1 << 20
 
 
-def _is_diagonal(t):
-    """Are all off-diagonal entries of (sets, n, n) exactly zero and the diagonals finite?  (NumPy)"""
+def _is_diagonal(t, rows=None):
+    """Are all off-diagonal entries of (sets, n, n) (of the first ``rows`` rows) exactly zero and the
+    diagonals finite?  (NumPy)"""
     d = np.diagonal(t, axis1=-2, axis2=-1)
     if not np.all(np.isfinite(d)):
         return False
     step = max(1, (1 << 14) // max(1, t.shape[-1]))
     return all(np.count_nonzero(t[:, r:r + step]) == np.count_nonzero(d[:, r:r + step])
-               for r in range(0, t.shape[-1], step))
+               for r in range(0, t.shape[-1] if rows is None else rows, step))
 
 
 def _look(T):
@@ -114,9 +121,9 @@ def fold_jump_operators(H, c_ops, dev=None):
     lops (S,Kd,N,N) or None.  A jump operator is *diagonal* when every off-diagonal
     entry of every set is exactly zero and its diagonal is finite.
 
-    Host operators are looked at on the host, operators on the GPU in stacks of up to ``_STACK_BYTES`` with
-    one read-back for all of them; of the diagonal ones only the diagonals are kept, so many of them cost
-    no memory.  (A product, a test and a synchronisation per
+    Small host operators are looked at on the host, large ones and operators on the GPU in stacks of up to
+    ``_STACK_BYTES`` there (those on the GPU with one read-back for all); of the diagonal ones only the
+    diagonals are kept, so many of them cost no memory.  (A product, a test and a synchronisation per
     operator took 110 us each: 3.4 of 5.0 ms of a two-time correlation with 16 on-site operators.)
     """
     dev = dev or device()
@@ -128,6 +135,15 @@ def fold_jump_operators(H, c_ops, dev=None):
     S, n = Ht.shape[0], Ht.shape[-1]
     ops, diag = {}, {}                         # dense (or not looked at yet), and diagonals, by number
     groups = {}                                # GPU operators by their number of sets
+    large = {}                                 # large host operators by number of sets: a stack, its numbers
+
+    def look_at_large(sets):
+        T, ks = large.pop(sets)
+        T = T[:, :len(ks)]
+        d, off = _look(T)
+        for x, (k, dense) in enumerate(zip(ks, off.tolist())):
+            (ops if dense else diag)[k] = (T if dense else d)[:, x]
+
     c_ops = list(c_ops or [])
 
     def take(k, c):
@@ -142,13 +158,24 @@ def fold_jump_operators(H, c_ops, dev=None):
         if isinstance(t, torch.Tensor):
             ops[k] = t
             groups.setdefault(sets, []).append(k)
-        elif not _is_diagonal(t):
+        elif not _is_diagonal(t, None if t.nbytes < _LOOK_BYTES else 1):
             ops[k] = t
-        else:
+        elif t.nbytes < _LOOK_BYTES:
             diag[k] = np.diagonal(t, axis1=-2, axis2=-1).copy()
+        else:
+            if sets not in large:
+                room = min(len(c_ops) - k, max(1, _STACK_BYTES // t.nbytes))
+                large[sets] = torch.empty((sets, room, n, n), dtype=torch.complex128, device=dev), []
+            T, ks = large[sets]
+            T[:, len(ks)] = torch.as_tensor(t)
+            ks.append(k)
+            if len(ks) == T.shape[1]:
+                look_at_large(sets)
 
     for k, c in enumerate(c_ops):
         take(k, c)
+    for sets in list(large):
+        look_at_large(sets)
     looked, stacks = [], {}
     for sets, ks in groups.items():
         many = max(1, _STACK_BYTES // max(1, 16 * sets * n * n))
@@ -173,7 +200,7 @@ def fold_jump_operators(H, c_ops, dev=None):
     def stack(xs):                                          # (1 or S, K, ...)
         sets = max(x.shape[0] for x in xs)
         mixed = len({isinstance(x, torch.Tensor) for x in xs}) > 1
-        if mixed or 16 * sets * len(xs) * int(np.prod(xs[0].shape[1:])) > _STACK_BYTES:
+        if mixed or 16 * sets * int(np.prod(xs[0].shape[1:])) >= _COPY_BYTES:
             out = torch.empty((sets, len(xs), *xs[0].shape[1:]), dtype=torch.complex128, device=dev)
             for k, x in enumerate(xs):
                 out[:, k] = x if isinstance(x, torch.Tensor) else torch.as_tensor(x)

@@ -11,12 +11,13 @@ import test_fold
 torch = pytest.importorskip("torch")
 
 
-def _limits(monkeypatch, stack):
+def _limits(monkeypatch, stack, copy, look):
     from lime_amd import propagator
-    monkeypatch.setattr(propagator, "_STACK_BYTES", stack)
+    for name, value in (("_STACK_BYTES", stack), ("_COPY_BYTES", copy), ("_LOOK_BYTES", look)):
+        monkeypatch.setattr(propagator, name, value)
 
 
-LIMITS = [(1,), (16 * 2 * 36,), (1200,)]
+LIMITS = [(1, 1, 1), (16 * 2 * 36, 1, 1 << 30), (1200, 1 << 30, 1), (1 << 30, 1, 1), (1200, 600, 400)]
 
 
 @pytest.mark.parametrize("limits", LIMITS)
@@ -55,6 +56,20 @@ def test_sparse_diagonal_operators_are_not_held_as_matrices():
     peak = tracemalloc.get_traced_memory()[1]
     tracemalloc.stop()
     assert peak < 8 * 16 * n * n, peak / (16 * n * n)            # a few matrices, not 48
+
+
+@pytest.mark.parametrize("look", [1, 1 << 30])
+def test_the_order_of_the_operators_is_kept(look, monkeypatch):
+    """Dense operators found on the host, on the GPU and in the first rows or past them."""
+    from lime_amd.propagator import fold_jump_operators
+    _limits(monkeypatch, 3 * 16 * 25, 1, look)
+    n = 5
+    ops = [(k + 1) * np.eye(n, dtype=complex) for k in range(9)]
+    for k, at in ((1, (4, 0)), (3, (0, 4)), (4, (2, 1)), (8, (4, 3))):
+        ops[k][at] = 1j
+    _, D, L = fold_jump_operators(np.zeros((n, n)), ops, torch.device("cpu"))
+    assert np.array_equal(L[0].numpy(), np.stack([ops[k] for k in (1, 3, 4, 8)]))
+    assert np.array_equal(D[0].numpy(), np.full((n, n), sum((k + 1) ** 2 for k in (0, 2, 5, 6, 7))))
 
 
 @pytest.mark.gpu
