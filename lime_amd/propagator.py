@@ -75,22 +75,22 @@ def _on_host(x):
 
 def as_c128_stack(xs, dev, dim=0):
     """Operators of one shape -> one complex128 tensor on ``dev`` (stacked along ``dim``), in
-    one copy where they all come from the host (a copy each costs more than the data of small
-    operators)."""
-    host = [_on_host(x) for x in xs]
-    if all(h is not None for h in host) and len({h.shape for h in host}) == 1:
-        return torch.as_tensor(np.stack(host, axis=dim), device=dev)
-    return torch.stack([as_c128(x, dev) for x in xs], dim=dim)
+    one copy where they all come from the host and are small (a copy each costs more than the data)."""
+    host = []
+    for x in xs:
+        h = _on_host(x)
+        if h is None or h.nbytes >= _LARGE_BYTES or (host and h.shape != host[0].shape):
+            return torch.stack([as_c128(x, dev) for x in xs], dim=dim)
+        host.append(h)
+    return torch.as_tensor(np.stack(host, axis=dim), device=dev) if host else torch.stack([], dim=dim)
 
 
 #: operators are looked at on the GPU this many bytes at a time (at least one operator)
 _STACK_BYTES = 64 << 20
-#: host operators of this size go to the GPU one by one, smaller ones stacked on the host: a copy costs
-#: 25 us, a stack 0.25 us a KB (16 of n = 512: 4.9 / 9.5 ms)
-_COPY_BYTES = 256 << 10
-#: host operators of this size are looked at on the GPU, past their first rows: the host reads 11 GB/s, the
-#: copies take 20 (32 diagonal ones of n = 1024: 49 ms on the host, 25 on the GPU)
-_LOOK_BYTES = 1 << 20
+#: host operators of this size go to the GPU one by one, smaller ones stacked on the host (ms stacked / one by
+#: one: 16 of n = 64 0.09 / 0.27, n = 256 0.89 / 0.91, n = 512 6.8 / 2.9), and past their first rows they are
+#: looked at there (32 diagonal ones of n = 1024: 49 ms on the host, 22 on the GPU; 64 of n = 512 25 / 14)
+_LARGE_BYTES = 1 << 20
 
 
 def _is_diagonal(t, rows=None):
@@ -158,9 +158,9 @@ def fold_jump_operators(H, c_ops, dev=None):
         if isinstance(t, torch.Tensor):
             ops[k] = t
             groups.setdefault(sets, []).append(k)
-        elif not _is_diagonal(t, None if t.nbytes < _LOOK_BYTES else 1):
+        elif not _is_diagonal(t, None if t.nbytes < _LARGE_BYTES else 1):
             ops[k] = t
-        elif t.nbytes < _LOOK_BYTES:
+        elif t.nbytes < _LARGE_BYTES:
             diag[k] = np.diagonal(t, axis1=-2, axis2=-1).copy()
         else:
             if sets not in large:
@@ -200,7 +200,7 @@ def fold_jump_operators(H, c_ops, dev=None):
     def stack(xs):                                          # (1 or S, K, ...)
         sets = max(x.shape[0] for x in xs)
         mixed = len({isinstance(x, torch.Tensor) for x in xs}) > 1
-        if mixed or 16 * sets * int(np.prod(xs[0].shape[1:])) >= _COPY_BYTES:
+        if mixed or 16 * sets * int(np.prod(xs[0].shape[1:])) >= _LARGE_BYTES:
             out = torch.empty((sets, len(xs), *xs[0].shape[1:]), dtype=torch.complex128, device=dev)
             for k, x in enumerate(xs):
                 out[:, k] = x if isinstance(x, torch.Tensor) else torch.as_tensor(x)

@@ -11,13 +11,13 @@ import test_fold
 torch = pytest.importorskip("torch")
 
 
-def _limits(monkeypatch, stack, copy, look):
+def _limits(monkeypatch, stack, large):
     from lime_amd import propagator
-    for name, value in (("_STACK_BYTES", stack), ("_COPY_BYTES", copy), ("_LOOK_BYTES", look)):
+    for name, value in (("_STACK_BYTES", stack), ("_LARGE_BYTES", large)):
         monkeypatch.setattr(propagator, name, value)
 
 
-LIMITS = [(1, 1, 1), (16 * 2 * 36, 1, 1 << 30), (1200, 1 << 30, 1), (1 << 30, 1, 1), (1200, 600, 400)]
+LIMITS = [(1, 1), (16 * 2 * 36, 1 << 30), (1200, 1), (1 << 30, 1), (1200, 400)]
 
 
 @pytest.mark.parametrize("limits", LIMITS)
@@ -58,11 +58,11 @@ def test_sparse_diagonal_operators_are_not_held_as_matrices():
     assert peak < 8 * 16 * n * n, peak / (16 * n * n)            # a few matrices, not 48
 
 
-@pytest.mark.parametrize("look", [1, 1 << 30])
-def test_the_order_of_the_operators_is_kept(look, monkeypatch):
+@pytest.mark.parametrize("large", [1, 1 << 30])
+def test_the_order_of_the_operators_is_kept(large, monkeypatch):
     """Dense operators found on the host, on the GPU and in the first rows or past them."""
     from lime_amd.propagator import fold_jump_operators
-    _limits(monkeypatch, 3 * 16 * 25, 1, look)
+    _limits(monkeypatch, 3 * 16 * 25, large)
     n = 5
     ops = [(k + 1) * np.eye(n, dtype=complex) for k in range(9)]
     for k, at in ((1, (4, 0)), (3, (0, 4)), (4, (2, 1)), (8, (4, 3))):
@@ -97,3 +97,18 @@ def test_memory_on_the_gpu(dense):
     # a stack and its mask, the dense operators once, a few matrices
     assert peak < 1.2 * _STACK_BYTES + (dense + 10) * one, peak / one
     assert out[1] is not None and (out[2] is not None) == (dense > 0)
+
+
+@pytest.mark.parametrize("large", [1, 16 * 9, 1 << 30])
+def test_operators_of_any_size_stack_alike(large, monkeypatch):
+    from lime_amd.propagator import as_c128_stack
+    _limits(monkeypatch, 1 << 20, large)
+    rng, cpu = np.random.default_rng(4), torch.device("cpu")
+    c = [rng.standard_normal((3, 3)) + 1j * rng.standard_normal((3, 3)) for _ in range(4)]
+    xs = [c[0], c[1].tolist(), sp.csr_matrix(c[2]), torch.as_tensor(c[3]).conj()]
+    for dim in (0, 1):
+        got = as_c128_stack(xs, cpu, dim=dim)
+        assert got.is_contiguous() and np.array_equal(got.numpy(), np.stack([*c[:3], c[3].conj()], axis=dim))
+    for bad in ([], [c[0], c[1][:2]]):
+        with pytest.raises(RuntimeError):
+            as_c128_stack(bad, cpu)
