@@ -16,6 +16,16 @@ __device__ __forceinline__ floatx4 mfma_f32(float a, float b, floatx4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
+// A barrier that the waves of a workgroup may reach from different places of the code.  s_barrier counts
+// arriving waves, not places, so this is sound as long as every wave of the workgroup passes the
+// same number of them; __syncthreads() promises that only where all threads reach the same call.  The
+// fences are what __syncthreads() has around it (LDS and global writes of the workgroup are seen after it).
+__device__ __forceinline__ void wave_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
 // DPP lane moves (no LDS round trip).  CTRL: 0xB1 = quad_perm(1,0,3,2), lane l reads
 // l ^ 1; 0x4E = quad_perm(2,3,0,1), l ^ 2; 0x141 = row_half_mirror, l reads the lane at
 // the mirrored position of its 8-lane half-row; 0x140 = row_mirror, of its 16-lane row.

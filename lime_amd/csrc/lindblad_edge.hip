@@ -235,8 +235,9 @@ __device__ __forceinline__ void edge_tr(const float2* sT, const float2* sR, int 
   }
 }
 
-// The run of one wave: a core tile (ROLE 0) or the parts in ROLE of 64 edge outputs.  Every form
-// passes the same barriers.  A wave of Re C holds the imaginary part of the state and one of Im C the
+// The run of one wave: a core tile (ROLE 0) or the parts in ROLE of 64 edge outputs.  The forms are
+// different code with the same number of barriers (one, then 4 (n_dense + 1) a step and one more with
+// renormalisation).  A wave of Re C holds the imaginary part of the state and one of Im C the
 // real part (k = -i C).
 template <int M, bool DRV, bool REC, int ROLE>
 __device__ __forceinline__ void edge_run(const ResidentArgs& a, int b, int tid, int w, int e0, const EdgeLds<M>& m,
@@ -295,7 +296,7 @@ __device__ __forceinline__ void edge_run(const ResidentArgs& a, int b, int tid, 
       put_s(m.s0, v, (float)rx[v], (float)ry[v]);
     }
   }
-  __syncthreads();
+  wave_barrier();
 
   const double dt = a.dt;
   int ph = 0;
@@ -326,7 +327,7 @@ __device__ __forceinline__ void edge_run(const ResidentArgs& a, int b, int tid, 
         const float2 t = edge_l<M>(m.l, sS, ri, j);
         if (own) m.t0[i0 * P + j] = t;
       }
-      __syncthreads();
+      wave_barrier();
       // driven: every wave is past its products with H_eff; the next step's loads leave here and
       // are stored after the step's last products
       float2 hn[G::NEXT];
@@ -350,7 +351,7 @@ __device__ __forceinline__ void edge_run(const ResidentArgs& a, int b, int tid, 
           const float2 t = edge_l<M>(L, sS, ri, j);
           if (own) Tn[i0 * P + j] = t;
         }
-        __syncthreads();
+        wave_barrier();
       }
       const float2 *Tk = kk & 1 ? m.t1 : m.t0, *R = m.r + kk * G::MAT;
       if constexpr (CORE) core_tr<M, false>(Tk, R, nullptr, nullptr, ri, j, lg, cr, ci, tr, ti);
@@ -370,7 +371,7 @@ __device__ __forceinline__ void edge_run(const ResidentArgs& a, int b, int tid, 
             put_s(sN, v, (float)(rx[v] + cnext * (double)kr), (float)(ry[v] + cnext * (double)ki));
           }
         }
-        __syncthreads();
+        wave_barrier();
         ph ^= 1;
         continue;
       }
@@ -396,7 +397,7 @@ __device__ __forceinline__ void edge_run(const ResidentArgs& a, int b, int tid, 
           for (int v = 0; v < NV; ++v)
             if (own && i0 + v == j) m.diag[j] = rx[v];
         }
-        __syncthreads();
+        wave_barrier();
         if constexpr (STATE) {
           double tot = 0.0;
 #pragma unroll
@@ -453,7 +454,7 @@ __device__ __forceinline__ void edge_run(const ResidentArgs& a, int b, int tid, 
           }
         }
       }
-      __syncthreads();   // S (and H_eff) of the next step and the record partials are complete
+      wave_barrier();   // S (and H_eff) of the next step and the record partials are complete
       ph ^= 1;
       // the record's sums go to the last wave (at three parts it holds no state)
       if constexpr (REC && EDGE_T) {

@@ -165,10 +165,10 @@ __device__ __forceinline__ void gemm_term(const typename CT<R>::C* __restrict__ 
   pa.load(n, n - kb, tid);
   pb.load(n, n - kb, tid);
   const auto stage = [&](int k0) {
-    __syncthreads();                          // previous panel fully consumed
+    wave_barrier();                           // previous panel fully consumed
     pa.store(sA, n - k0, tid);
     pb.store(sB, n - k0, tid);
-    __syncthreads();
+    wave_barrier();
     if (k0 + KW < ke) {                       // prefetch the next panel into registers
       pa.load(n, n - k0 - KW, tid);
       pb.load(n, n - k0 - KW, tid);
@@ -199,7 +199,8 @@ __device__ __forceinline__ void gemm_term(const typename CT<R>::C* __restrict__ 
   // whole panels of blocks inside the operator: one basic block a panel, its fragment reads ahead
   // of the products (a test per k-step left every read's latency in front of its three MFMAs).  A
   // loop of its own: a branch inside one loop makes the compiler keep two sets of accumulators and
-  // copy between them.  FP64 keeps one loop: the fragments' registers cost it waves.  us per RK4
+  // copy between them.  Waves at the operator's edge take all their panels in the loop below: two
+  // barriers a panel in either, so every wave passes the same number.  FP64 keeps one loop: the fragments' registers cost it waves.  us per RK4
   // step, FP32, tested / here: 16 x n = 512 with 16 jump operators (64-tiles) 14360 / 13630, one of
   // them (32) 1686 / 1519, 16 x n = 256 with 4 (32) 732 / 681, 16 x n = 129 69 / 65.
   if (sizeof(R) == 4 && all_live) {
@@ -759,7 +760,8 @@ __device__ __forceinline__ void gemm_term_bf3(const void* __restrict__ A, const 
   int k0 = kb;
   // WHOLE: whole panels of blocks inside the operator: loads at one wave-uniform address plus 32-bit
   // offsets formed once (as Panel above), and one basic block of products, the accumulators in turn so
-  // that no MFMA waits for the one before it (each accumulator's own order is that of the tested loop)
+  // that no MFMA waits for the one before it (each accumulator's own order is that of the tested loop).
+  // Both loops pass two barriers a panel: waves that take different ones pass the same number.
   if (WHOLE && all_live && (MODE != PLAIN || n % 2 == 0)) {
     FastRows<TILE, APS> fa;
     FastRows<MODE == PLAIN ? KB : TILE, BPS, MODE == PLAIN ? TILE : KB> fb;
@@ -773,10 +775,10 @@ __device__ __forceinline__ void gemm_term_bf3(const void* __restrict__ A, const 
     if (PF && k0 < ke && k0 + KB <= n) load_fast();
     for (; k0 < ke && k0 + KB <= n; k0 += KB) {
       if constexpr (!PF) load_fast();
-      __syncthreads();
+      wave_barrier();
       fa.template store<PP, false>(sA, tid);
       fb.template store<MODE == PLAIN ? PB : PP, MODE == NEG_AH>(sB, tid);
-      __syncthreads();
+      wave_barrier();
       if constexpr (PF) {
         if (k0 + KB < ke && k0 + 2 * KB <= n) load_fast();
       }
@@ -809,11 +811,11 @@ __device__ __forceinline__ void gemm_term_bf3(const void* __restrict__ A, const 
   if constexpr (PF) load_panel(k0);
   for (; k0 < ke; k0 += KB) {
     if constexpr (!PF) load_panel(k0);
-    __syncthreads();                          // previous panel fully consumed
+    wave_barrier();                          // previous panel fully consumed
     ra.template store<false>(sA, tid);
     if constexpr (MODE == PLAIN) store_pairs<KB, TILE, PB, false>(sB, rp, tid);
     else rb.template store<MODE == NEG_AH>(sB, tid);
-    __syncthreads();
+    wave_barrier();
     if constexpr (PF) {
       if (k0 + KB < ke) load_panel(k0 + KB);  // prefetch the next panel into registers
     }
