@@ -1019,29 +1019,29 @@ hipError_t launch_rec2(const ResidentArgs& a, size_t lds, hipStream_t stream) {
     static_assert(MINW <= 5, "the budget of the driven kernels");
     return a.op_pitch > 0 ? launch_dense<NB, W, BPW, MINW, true>(a, lds, stream)
                           : launch_dense<NB, W, BPW, MINW, false>(a, lds, stream);
-  }
-  if constexpr (!DENSE && (BPW == 1 || NB == 5) && !BRD && DB && NB >= 2) {
-    if (a.heff_step <= 0) {
-      switch (cdiv(a.n, 4)) {
+  } else {
+    if (a.heff_step > 0) {
+      // driven systems run the default shape; at 6 waves per SIMD the step's extra addresses spill
+      // two registers, and the few operators of a driven call do not need the occupancy
+      constexpr Shape first = (BRD ? kBorderShapes : kShapes)[NB][0];
+      constexpr int MW = MINW > 5 ? 5 : MINW;
+      if constexpr (W == first.w && BPW == first.bpw)
+        return launch_kernel(lindblad_rk4_resident_driven<NB, W, BPW, MW, DENSE, BRD, DB, false>, a, W, lds, stream);
+      return hipErrorInvalidValue;
+    }
+    if constexpr (!DENSE && (BPW == 1 || NB == 5) && !BRD && DB && NB >= 2) {
+      switch (cdiv(a.n, 4)) {                 // every length of the padded size is built in
         case k_steps<NB, -1>(): return launch_plain<NB, W, BPW, MINW, k_steps<NB, -1>()>(a, lds, stream);
         case k_steps<NB, 0>(): return launch_plain<NB, W, BPW, MINW, k_steps<NB, 0>()>(a, lds, stream);
         case k_steps<NB, 1>(): return launch_plain<NB, W, BPW, MINW, k_steps<NB, 1>()>(a, lds, stream);
         case k_steps<NB, 2>(): return launch_plain<NB, W, BPW, MINW, k_steps<NB, 2>()>(a, lds, stream);
+        default: return hipErrorInvalidValue;
       }
+    } else {
+      return rec ? launch_kernel(lindblad_rk4_resident<NB, W, BPW, MINW, DENSE, true, BRD, DB>, a, W, lds, stream)
+                 : launch_kernel(lindblad_rk4_resident<NB, W, BPW, MINW, DENSE, false, BRD, DB>, a, W, lds, stream);
     }
   }
-  if (a.heff_step > 0) {
-    // driven systems run the default shape; at 6 waves per SIMD the step's extra addresses spill
-    // two registers, and the few operators of a driven call do not need the occupancy
-    constexpr Shape first = (BRD ? kBorderShapes : kShapes)[NB][0];
-    constexpr int MW = MINW > 5 ? 5 : MINW;
-    if constexpr (W == first.w && BPW == first.bpw) {
-      return launch_kernel(lindblad_rk4_resident_driven<NB, W, BPW, MW, DENSE, BRD, DB, false>, a, W, lds, stream);
-    }
-    return hipErrorInvalidValue;
-  }
-  return rec ? launch_kernel(lindblad_rk4_resident<NB, W, BPW, MINW, DENSE, true, BRD, DB>, a, W, lds, stream)
-             : launch_kernel(lindblad_rk4_resident<NB, W, BPW, MINW, DENSE, false, BRD, DB>, a, W, lds, stream);
 }
 
 template <int NB, int W, int BPW, int MINW, bool DENSE, bool BRD>
