@@ -96,12 +96,13 @@ _LARGE_BYTES = 1 << 20
 def _is_diagonal(t, rows=None):
     """Are all off-diagonal entries of (sets, n, n) (of the first ``rows`` rows) exactly zero and the
     diagonals finite?  (NumPy)"""
-    d = np.diagonal(t, axis1=-2, axis2=-1)
-    if not np.all(np.isfinite(d)):
-        return False
-    step = max(1, (1 << 14) // max(1, t.shape[-1]))
-    return all(np.count_nonzero(t[:, r:r + step]) == np.count_nonzero(d[:, r:r + step])
-               for r in range(0, t.shape[-1] if rows is None else rows, step))
+    d = t.diagonal(0, -2, -1)
+    if t.size <= 1 << 14:
+        return np.count_nonzero(t) == np.count_nonzero(d) and bool(np.isfinite(d).all())
+    step = max(1, (1 << 14) // t.shape[-1])
+    return bool(np.isfinite(d).all()) and all(
+        np.count_nonzero(t[:, r:r + step]) == np.count_nonzero(d[:, r:r + step])
+        for r in range(0, t.shape[-1] if rows is None else rows, step))
 
 
 def _look(T):
@@ -150,7 +151,7 @@ def fold_jump_operators(H, c_ops, dev=None):
         t = _on_host(c)
         t = c if t is None else t
         t = t[None] if t.ndim == 2 else t
-        if tuple(t.shape[-2:]) != (n, n):
+        if t.shape[-2:] != (n, n):
             raise ValueError(f"c_ops[{k}] has shape {tuple(t.shape)}, expected (..., {n}, {n})")
         sets = t.shape[0]
         if t.ndim != 3 or sets not in (1, S):
@@ -158,10 +159,12 @@ def fold_jump_operators(H, c_ops, dev=None):
         if isinstance(t, torch.Tensor):
             ops[k] = t
             groups.setdefault(sets, []).append(k)
-        elif not _is_diagonal(t, None if t.nbytes < _LARGE_BYTES else 1):
+            return
+        small = t.nbytes < _LARGE_BYTES
+        if not _is_diagonal(t, None if small else 1):
             ops[k] = t
-        elif t.nbytes < _LARGE_BYTES:
-            diag[k] = np.diagonal(t, axis1=-2, axis2=-1).copy()
+        elif small:
+            diag[k] = t.diagonal(0, -2, -1).copy()
         else:
             if sets not in large:
                 room = min(len(c_ops) - k, max(1, _STACK_BYTES // t.nbytes))
@@ -199,15 +202,16 @@ def fold_jump_operators(H, c_ops, dev=None):
 
     def stack(xs):                                          # (1 or S, K, ...)
         sets = max(x.shape[0] for x in xs)
-        mixed = len({isinstance(x, torch.Tensor) for x in xs}) > 1
-        if mixed or 16 * sets * int(np.prod(xs[0].shape[1:])) >= _LARGE_BYTES:
-            out = torch.empty((sets, len(xs), *xs[0].shape[1:]), dtype=torch.complex128, device=dev)
-            for k, x in enumerate(xs):
-                out[:, k] = x if isinstance(x, torch.Tensor) else torch.as_tensor(x)
-            return out
-        wide = [x.expand(sets, *x.shape[1:]) if isinstance(x, torch.Tensor) else
-                np.broadcast_to(x, (sets, *x.shape[1:])) for x in xs]
-        return as_c128_stack(wide, dev, dim=1)
+        on_host = [not isinstance(x, torch.Tensor) for x in xs]
+        if all(on_host) and 16 * sets * int(np.prod(xs[0].shape[1:])) < _LARGE_BYTES:
+            wide = [x if x.shape[0] == sets else np.broadcast_to(x, (sets, *x.shape[1:])) for x in xs]
+            return torch.as_tensor(np.stack(wide, axis=1), device=dev)
+        if not any(on_host):
+            return torch.stack([x.to(device=dev, dtype=torch.complex128).expand(sets, *x.shape[1:]) for x in xs], dim=1)
+        out = torch.empty((sets, len(xs), *xs[0].shape[1:]), dtype=torch.complex128, device=dev)
+        for k, x in enumerate(xs):
+            out[:, k] = torch.as_tensor(x)
+        return out
 
     if dense:
         L = stacks[tuple(dense)] if stacks else stack([ops[k] for k in dense])
