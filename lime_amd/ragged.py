@@ -151,6 +151,8 @@ class RaggedLindblad:
         if tune:
             from . import autotune
             autotune.tune_ragged(self, dt_tune, verbose=verbose)
+        if self.variant >= self.variants():       # a choice from the cache was not timed here: a first step
+            self._tile_lists(TILE_EDGES[self.variant - self.variants()])     # may be one that is captured
 
     def variants(self):
         """Launch shapes of the persistent kernel."""

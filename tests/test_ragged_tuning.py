@@ -119,3 +119,32 @@ def test_a_launch_that_is_not_offered_is_refused(variant, max_groups):
     rb.sizes, rb.kd, rb.cost, rb._lists, rb.dev = np.array([4]), np.array([0]), np.array([64.0]), {}, "cpu"
     with pytest.raises(_lib.LimeError, match="variant"):
         rb.step(0.01, 1, stream=SimpleNamespace(cuda_stream=0))
+
+
+@pytest.mark.gpu
+def test_the_first_step_of_a_batch_with_a_cached_choice_can_be_captured(cache):
+    """The workgroup lists are there before the first step: a copy to the GPU cannot be captured."""
+    from lime_amd import autotune
+    from lime_amd.ragged import RaggedLindblad
+    rng = np.random.default_rng(3)
+    inst = []
+    for n in (8, 33, 70):
+        x = rng.standard_normal((n, n))
+        inst.append(dict(H=(x + x.T) / n + 0j, c_ops=[x / n ** 2], dephasing=0.01, rho0=np.eye(n) / n + 0j))
+    want = RaggedLindblad(inst, tune=False)
+    for variant in (want.variants(), want.variants() + 1):
+        want.variant = variant
+        want.step(0.02, 1)                             # the kernels are loaded
+        want.rho.copy_(RaggedLindblad(inst, tune=False).rho)
+        cache[autotune.ragged_key(want)] = {"variant": variant}
+        rb = RaggedLindblad(inst)
+        assert rb.variant == variant and len(rb._lists) == 1
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            rb.step(0.02, 2)
+        for _ in range(3):
+            g.replay()
+            want.step(0.02, 2)
+            torch.cuda.synchronize()
+            assert torch.equal(rb.rho, want.rho)
