@@ -58,3 +58,23 @@ def test_per_phase_launches_equal_the_persistent_launch_eager_and_replayed():
         want.step(0.02, 2)
         assert torch.equal(rb.rho, want.rho), v
     assert RaggedLindblad(inst, tune=False, max_groups=1).launches() == ref.variants()
+
+
+@pytest.mark.gpu
+def test_a_run_of_many_steps_captures_a_bounded_graph():
+    torch = pytest.importorskip("torch")
+    from lime_amd.ragged import GRAPH_STEPS, RaggedLindblad
+    inst = _instances(6)[2:7]
+    steps = 2 * GRAPH_STEPS + 5
+    for v in (5, 6):
+        want, rb = (RaggedLindblad(inst, tune=False) for _ in range(2))
+        want.run(0.005, steps)
+        assert want.graph_steps == steps               # the persistent launch is one node
+        rb.variant = v
+        assert rb.variants() <= v < rb.launches()
+        rb.run(0.005, steps)
+        assert rb.graph_steps == GRAPH_STEPS
+        assert torch.equal(rb.rho, want.rho)
+        rb.run(0.005, 3, chunk=3)
+        want.run(0.005, 3)
+        assert rb.graph_steps == 3 and torch.equal(rb.rho, want.rho)
