@@ -224,6 +224,8 @@ class RaggedLindblad:
         """Advance every instance by ``nsteps`` steps by replaying the captured launch(es): all steps in
         one replay, or with a launch per phase (8 a step) ``GRAPH_STEPS`` of them, unless ``chunk`` says
         how many."""
+        if nsteps < 1:
+            return
         whole = nsteps if self.variant < self.variants() else min(nsteps, GRAPH_STEPS)
         chunk = int(chunk or whole)
         if self.graph is None or self.graph_steps != chunk or self.graph_dt != dt:
@@ -305,6 +307,8 @@ class RaggedClasses:
 
     def run(self, dt, nsteps, chunk=None):
         """Advance every instance by ``nsteps`` steps by replaying the captured graph."""
+        if nsteps < 1:
+            return
         chunk = int(chunk or nsteps)
         if self.graph is None or self.graph_steps != chunk or self.graph_dt != dt:
             self.capture(dt, chunk)

@@ -78,3 +78,9 @@ def test_a_run_of_many_steps_captures_a_bounded_graph():
         rb.run(0.005, 3, chunk=3)
         want.run(0.005, 3)
         assert rb.graph_steps == 3 and torch.equal(rb.rho, want.rho)
+
+
+def test_a_run_of_no_steps_ends():
+    from lime_amd.ragged import RaggedClasses, RaggedLindblad
+    for cls in (RaggedLindblad, RaggedClasses):
+        assert object.__new__(cls).run(0.01, 0) is None
