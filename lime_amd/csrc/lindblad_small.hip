@@ -9,7 +9,9 @@
 // stage, none across waves for n <= 8).
 //
 // The order of the products is the resident kernel's: the FP32 MFMA adds its four products one
-// after the other, each rounded like an FMA, so the results are the same bits as on the tiles.
+// after the other, each rounded like an FMA, so the results are the same bits as on the tiles.  The FP64 trace
+// of a renormalisation too: its elements lie on other lanes for n <= 8, but pair up in the same tree
+// (n = 1 .. 8, with and without, against a build that ran them on the tiles).
 #include "common.hpp"
 #include "lindblad_resident_decl.hpp"
 
