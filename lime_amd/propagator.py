@@ -29,6 +29,11 @@ def device():
     return torch.device("cuda", torch.cuda.current_device())
 
 
+def _as_tensor(a):
+    """A NumPy array as a CPU tensor (torch takes no negative strides)."""
+    return torch.as_tensor(a if min(a.strides, default=0) >= 0 else a.copy())
+
+
 def as_c128(x, dev):
     """Array-like or tensor -> contiguous complex128 tensor on ``dev``."""
     if isinstance(x, torch.Tensor):
@@ -37,7 +42,7 @@ def as_c128(x, dev):
     else:
         if hasattr(x, "toarray"):          # scipy.sparse
             x = x.toarray()
-        t = torch.as_tensor(np.asarray(x, dtype=np.complex128), device=dev)
+        t = _as_tensor(np.asarray(x, dtype=np.complex128)).to(dev)
     return t.contiguous()
 
 
@@ -170,7 +175,7 @@ def fold_jump_operators(H, c_ops, dev=None):
                 room = min(len(c_ops) - k, max(1, _STACK_BYTES // t.nbytes))
                 large[sets] = torch.empty((sets, room, n, n), dtype=torch.complex128, device=dev), []
             T, ks = large[sets]
-            T[:, len(ks)] = torch.as_tensor(t)
+            T[:, len(ks)] = _as_tensor(t)
             ks.append(k)
             if len(ks) == T.shape[1]:
                 look_at_large(sets)
@@ -210,7 +215,7 @@ def fold_jump_operators(H, c_ops, dev=None):
             return torch.stack([x.to(device=dev, dtype=torch.complex128).expand(sets, *x.shape[1:]) for x in xs], dim=1)
         out = torch.empty((sets, len(xs), *xs[0].shape[1:]), dtype=torch.complex128, device=dev)
         for k, x in enumerate(xs):
-            out[:, k] = torch.as_tensor(x)
+            out[:, k] = x if isinstance(x, torch.Tensor) else _as_tensor(x)
         return out
 
     if dense:

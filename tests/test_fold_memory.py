@@ -112,3 +112,17 @@ def test_operators_of_any_size_stack_alike(large, monkeypatch):
     for bad in ([], [c[0], c[1][:2]]):
         with pytest.raises(RuntimeError):
             as_c128_stack(bad, cpu)
+
+
+@pytest.mark.parametrize("large", [1, 1 << 30])
+def test_reversed_arrays(large, monkeypatch):
+    """NumPy views with negative strides, which torch does not take."""
+    from lime_amd.propagator import as_c128, as_c128_stack, fold_jump_operators
+    _limits(monkeypatch, 1 << 20, large)
+    cpu = torch.device("cpu")
+    a = np.arange(9.0).reshape(3, 3) + 1j
+    d = np.diag([1.0 + 0j, 2, 3])
+    assert np.array_equal(as_c128(a[::-1], cpu).numpy(), a[::-1])
+    assert np.array_equal(as_c128_stack([a[::-1], a.T], cpu).numpy(), np.stack([a[::-1], a.T]))
+    _, D, L = fold_jump_operators(a[:, ::-1], [d[::-1, ::-1], a[::-1]], cpu)
+    assert np.array_equal(L[0, 0].numpy(), a[::-1]) and np.array_equal(D[0].numpy(), np.outer([3, 2, 1], [3, 2, 1]))
